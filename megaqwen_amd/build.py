@@ -14,7 +14,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libmegaqwen_amd.so")
-SOURCES = ["mq_decode.hip", "mq_prefill.hip"]
+SOURCES = ["mq_decode.hip", "mq_prefill.hip", "mq_prefill_short.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 FLAGS = [

@@ -11,7 +11,8 @@
 //   -> gemm_nt (gate and up, SiLU(gate) * up epilogue) -> gemm_nt (down_proj, k split)
 //   -> resid_norm_rows (partials + residual, the next layer's input RMSNorm)
 // then lm_partial (final norm of the last row, tied LM head, per-block argmax) and
-// argmax_final. The GEMMs run on v_mfma_f32_16x16x32_bf16 with fp32 accumulation.
+// argmax_final. Prompts of at most 256 tokens run their layers in one launch instead
+// (mq_prefill_short.hip; the same bits). The GEMMs run on v_mfma_f32_16x16x32_bf16 with fp32 accumulation.
 //
 // The intermediates, the fp32 partial sums included, live in the caller's scratch
 // buffers (the reference's own argument list), so a launch allocates nothing.
@@ -28,6 +29,7 @@
 
 #include "megaqwen_amd.h"
 #include "mq_common.h"
+#include "mq_prefill_short.h"
 
 // Instrumentation hook of a tracing build: MQ_PF_STAMP(slot) marks a point of a kernel's
 // timeline; it compiles to nothing unless a tracing harness defines it first.
@@ -117,9 +119,9 @@ struct XcdMap {
 // prefill, same box: S = 300 1.779 -> 1.807 ms, 512 1.962 -> 1.992).
 constexpr int MAX_WARM = 5, NUM_CUS = 256;  // (MI355X: 8 XCDs of 32 CUs)
 // Prompts up to this length warm in gate/up (whole prefill, same box, without -> with the
-// warm-up: S = 64 1.465 -> 1.408 ms, 128 1.511 -> 1.474, 256 1.675 -> 1.639, 288 1.755 ->
-// 1.730, 352 1.804 -> 1.760, 384 1.839 -> 1.782; from 385 tokens gate/up has 192 tile
-// workgroups, and with the warm-up row S = 400 measured 1.794 -> 1.801, 512 1.930 -> 1.927)
+// warm-up: S = 288 1.755 -> 1.730 ms, 352 1.804 -> 1.760, 384 1.839 -> 1.782; from 385 tokens
+// gate/up has 192 tile workgroups, and with the warm-up row S = 400 measured 1.794 -> 1.801, 512
+// 1.930 -> 1.927)
 constexpr int WARM_MAX_S = 384;
 struct WarmSet {
   const uint16_t* w[MAX_WARM];  // weight matrices [n, k] bf16, in the order they are read
@@ -754,12 +756,6 @@ __device__ __forceinline__ void kv_chunk(const uint16_t* src, int k0, int klast,
 #define AWAIT(n) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(n) : "memory")
 #define ABAR() asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory")
 
-// TRIM (short prompts): the K loads, score products and exponentials stop at the block's
-// last key instead of covering all 512 (the skipped scores are masked, so the sums and
-// products are the same: same bits). Whole prefill, same box: S = 64 1.416 -> 1.368 ms, 128
-// 1.462 -> 1.429, 256 1.636 -> 1.621; at S = 512 the branches cost more than they save
-// (1.990 -> 2.015), so longer prompts keep the straight-line form.
-template <bool TRIM>
 __global__ void __launch_bounds__(64 * AW) attn_prefill(const uint16_t* q, const uint16_t* kc, const uint16_t* vc,
                                                        uint16_t* out, int S, int max_seq, float scale) {
   typedef short v4s __attribute__((ext_vector_type(4)));
@@ -816,7 +812,6 @@ __global__ void __launch_bounds__(64 * AW) attn_prefill(const uint16_t* q, const
 #pragma unroll
     for (int i = 0; i < AKB / ACK / 2; i++) {
       const int c = 2 * i + kpar;
-      if (TRIM && ACK * c >= nk) break;
       const int krow = min(kb0 + ACK * c + 16 * kw + r16, kb1 - 1);
 #pragma unroll
       for (int ks = 0; ks < 4; ks++) kf[i][ks] = ldw(K + (size_t)krow * HD + 32 * ks + 8 * kg);
@@ -825,7 +820,6 @@ __global__ void __launch_bounds__(64 * AW) attn_prefill(const uint16_t* q, const
 #pragma unroll
     for (int i = 0; i < AKB / ACK / 2; i++) {
       const int c = 2 * i + kpar;
-      if (TRIM && ACK * c >= nk) break;  // (the unwritten score columns are past nk)
       {
         const int row = 16 * kw + r16, key = kb0 + ACK * c + row;
 #pragma unroll
@@ -848,11 +842,10 @@ __global__ void __launch_bounds__(64 * AW) attn_prefill(const uint16_t* q, const
     // row are issued together and the reductions interleaved); lane takes keys lane + 64 u
     {
       float x[RPW][AKB / 64], mx[RPW], sum[RPW];
-      const int nu = TRIM ? (nk + 63) >> 6 : AKB / 64;  // 64-key columns read
 #pragma unroll
       for (int i = 0; i < RPW; i++)
 #pragma unroll
-        for (int u = 0; u < AKB / 64; u++) x[i][u] = u < nu ? s_sc[RPW * wv + i][lane + 64 * u] : -INFINITY;  // past nk: unused
+        for (int u = 0; u < AKB / 64; u++) x[i][u] = s_sc[RPW * wv + i][lane + 64 * u];
 #pragma unroll
       for (int i = 0; i < RPW; i++) {
         mx[i] = -INFINITY;
@@ -870,7 +863,6 @@ __global__ void __launch_bounds__(64 * AW) attn_prefill(const uint16_t* q, const
         // +0 leaves the sum unchanged; P.V reads s_p only below nk32)
 #pragma unroll
         for (int u = 0; u < AKB / 64; u++) {
-          if (u >= nu) break;  // (P.V reads s_p below nk32 <= 64 nu only)
           const int cc = lane + 64 * u;
           const float ev = exp_fast(x[i][u] - base);
           const float e = cc < nk ? ev : 0.f;
@@ -1707,13 +1699,6 @@ void gemm(GemmArgs g, int ntiles, hipStream_t stream, int split = 1, int xg = 0,
     gemm_nt<EPI, TM, TN, NST, KS, WM, WN><<<dim3(ntiles, ny, split), 64 * WM * WN, 0, stream>>>(ka);
   }
 }
-// Prompts of at most SHORT_S tokens fill few CUs with the tiles of S = 512 (gate/up 48 x 2
-// workgroups at S = 256), so they take smaller row tiles: q/k/v 32 x 128, gate/up 64 x 128
-// (32 x 128 up to 128 tokens, 64 x 64 up to 64), the k-split residual products 64 x 64 (32 x
-// 64 up to 128). Every tile sums its k range in the same order whatever its shape, so the
-// outputs are the same bits. Whole prefill, same box, with the warm-up (ms): S = 64 1.600 ->
-// 1.408, 96 1.644 -> 1.451, 128 1.699 -> 1.474, 192 1.706 -> 1.591, 256 1.780 -> 1.639.
-constexpr int SHORT_S = 256;
 static void gemm_qkv(GemmArgs g, hipStream_t stream) {
   // Long prompts: two heads a tile on sixteen waves (256 x 256, two stages; the epilogue stages
   // both heads through the ring as bf16), blockIdx order, the same bits as the one-head
@@ -1758,8 +1743,7 @@ static void gemm_qkv(GemmArgs g, hipStream_t stream) {
   // 99.3 us against blockIdx order, same-box medians)
   if (g.m >= 2048) gemm<EPI_QKN, 256, HD, 3, 1, 4, 2>(g, nt, stream, 1, 1, 4);
   else if (g.m >= 1024) gemm<EPI_QKN, 128, HD, 4, 1, 4, 2>(g, nt, stream);
-  else if (g.m > SHORT_S) gemm<EPI_QKN, 64, HD, 4, 1, 2, 4>(g, nt, stream);
-  else gemm<EPI_QKN, 32, HD, 4, 1, 2, 2>(g, nt, stream);
+  else gemm<EPI_QKN, 64, HD, 4, 1, 2, 4>(g, nt, stream);
 }
 // warm: the warm-up set of a prompt of at most WARM_MAX_S tokens, or null
 static void gemm_gate_up(GemmArgs g, hipStream_t stream, const WarmSet* warm = nullptr) {
@@ -1788,7 +1772,7 @@ static void gemm_gate_up(GemmArgs g, hipStream_t stream, const WarmSet* warm = n
   } else if (g.m > 512) {
     g.seg[0].ntiles = I / 64;
     gemm<EPI_SILU, 128, 128, 3, 1, 4, 4>(g, I / 64, stream, 1, 0, 1, warm);
-  } else if (g.m > SHORT_S) {
+  } else {
     // (257..512 tokens: 128 x 96 tiles on four waves, 64 column tiles, so 256 workgroups fill
     // the CUs where the 128 x 128 tiles leave 64 idle; same bits, whole prefill, same box:
     // S = 300 1.722 -> 1.714 ms, 384 1.774 -> 1.759, 512 1.923 -> 1.918; at 640 1.9x the
@@ -1796,15 +1780,6 @@ static void gemm_gate_up(GemmArgs g, hipStream_t stream, const WarmSet* warm = n
     // 1-3% slower)
     g.seg[0].ntiles = I / 48;
     gemm<EPI_SILU, 128, 96, 3, 1, 4, 1>(g, I / 48, stream, 1, 0, 1, warm);
-  } else if (g.m > 128) {
-    g.seg[0].ntiles = I / 64;
-    gemm<EPI_SILU, 64, 128, 3, 1, 2, 4>(g, I / 64, stream, 1, 0, 1, warm);
-  } else if (g.m > 64) {
-    g.seg[0].ntiles = I / 64;
-    gemm<EPI_SILU, 32, 128, 4, 1, 2, 2>(g, I / 64, stream, 1, 0, 1, warm);
-  } else {
-    g.seg[0].ntiles = I / 32;
-    gemm<EPI_SILU, 64, 64, 4, 1, 2, 2>(g, I / 32, stream, 1, 0, 1, warm);
   }
 }
 // Long prompts: o_proj / down_proj with the residual add in the epilogue (the four k quarters
@@ -1837,9 +1812,7 @@ static void gemm_residual(GemmArgs g, hipStream_t stream) {
     gemm<EPI_PART, 128, 128, 4, 1, 4, 2>(g, H / 128, stream, RES_SPLIT);
   } else {
     g.seg[0].ntiles = H / 64;
-    if (g.m > SHORT_S) gemm<EPI_PART, 128, 64, 4, 1, 4, 2>(g, H / 64, stream, RES_SPLIT);
-    else if (g.m > 128) gemm<EPI_PART, 64, 64, 4, 1, 2, 2>(g, H / 64, stream, RES_SPLIT);
-    else gemm<EPI_PART, 32, 64, 4, 1, 2, 2>(g, H / 64, stream, RES_SPLIT);
+    gemm<EPI_PART, 128, 64, 4, 1, 4, 2>(g, H / 64, stream, RES_SPLIT);
   }
 }
 
@@ -1904,6 +1877,26 @@ static int prefill_run(const int* input_token_ids, int* output_token_id, int seq
     if (e != hipSuccess && launch_err == hipSuccess) launch_err = e;
   };
   (void)hipGetLastError();  // clear an error left by an unrelated earlier call
+  auto lm_head = [&]() {
+    lm_partial<<<LMB, 256, 0, stream>>>(h + (size_t)(S - 1) * H, bf(final_norm_weight), bf(lm_head_weight),
+                                        B.final_bf16, B.final_f32, B.hidden_out, B.prenorm_out, B.bmv, B.bmi);
+    chk();
+    argmax_final<<<1, 256, 0, stream>>>(B.bmv, B.bmi, output_token_id, err);
+    chk();
+    return launch_err == hipSuccess ? MQ_OK : MQ_ERR_HIP;
+  };
+  if (S <= ps::SHORT_MAX_S) {
+    // every layer in one launch; its sync words live in scratch that it has no other use for
+    ps::ShortArgs A{};
+    A.S = S; A.num_layers = num_layers; A.max_seq = max_seq_len; A.scale = attn_scale;
+    A.h = h; A.q = qp; A.att = att; A.mid = mid;
+    A.kc = bfm(k_cache); A.vc = bfm(v_cache);
+    A.cos_t = bf(cos_table); A.sin_t = bf(sin_table);
+    A.sync = reinterpret_cast<uint32_t*>(parts.lo[0]); A.local = reinterpret_cast<uint32_t*>(nrm); A.err = err;
+    for (int l = 0; l < num_layers; l++) A.lw[l] = layer_weights[l];
+    const int rc = prefill_short_run(input_token_ids, bf(embed_weight), A, stream);
+    return rc == MQ_OK ? lm_head() : rc;
+  }
   embed_rows<<<S, 128, 0, stream>>>(input_token_ids, bf(embed_weight), h, err);
   chk();
   rmsnorm_rows<<<S, 64, 0, stream>>>(h, bf(layer_weights[0].input_layernorm_weight), nrm, S);
@@ -1929,10 +1922,8 @@ static int prefill_run(const int* input_token_ids, int* output_token_id, int seq
     else if (S > FLASH_MIN_S)
       attn_prefill_fa3<<<NKV * ((S + F3Q - 1) / F3Q), 64 * F3W, 0, stream>>>(qp, kcl, vcl, att, S, max_seq_len,
                                                                              attn_scale);
-    else if (S <= SHORT_S)
-      attn_prefill<true><<<NQ * ((S + AQ - 1) / AQ), 64 * AW, 0, stream>>>(qp, kcl, vcl, att, S, max_seq_len, attn_scale);
     else
-      attn_prefill<false><<<NQ * ((S + AQ - 1) / AQ), 64 * AW, 0, stream>>>(qp, kcl, vcl, att, S, max_seq_len, attn_scale);
+      attn_prefill<<<NQ * ((S + AQ - 1) / AQ), 64 * AW, 0, stream>>>(qp, kcl, vcl, att, S, max_seq_len, attn_scale);
     chk();
     GemmArgs go{};
     go.a = att; go.lda = QS; go.m = S; go.k = QS;
@@ -1988,12 +1979,7 @@ static int prefill_run(const int* input_token_ids, int* output_token_id, int seq
     }
     chk();
   }
-  lm_partial<<<LMB, 256, 0, stream>>>(h + (size_t)(S - 1) * H, bf(final_norm_weight), bf(lm_head_weight),
-                                      B.final_bf16, B.final_f32, B.hidden_out, B.prenorm_out, B.bmv, B.bmi);
-  chk();
-  argmax_final<<<1, 256, 0, stream>>>(B.bmv, B.bmi, output_token_id, err);
-  chk();
-  return launch_err == hipSuccess ? MQ_OK : MQ_ERR_HIP;
+  return lm_head();
 }
 
 extern "C" int launch_prefill_float(const int* input_token_ids, int* output_token_id, int seq_len,
