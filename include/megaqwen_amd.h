@@ -135,6 +135,11 @@ int mq_decode_layer(const void* hidden_in, void* hidden_out, const LDGLayerWeigh
                     const void* cos_table, const void* sin_table, void* k_cache, void* v_cache, int position,
                     int max_seq_len, float attn_scale, hipStream_t stream);
 
+/* Writes one layer's weight pointers (a HOST struct, copied during the call) to
+ * `device_layer` in device memory, ordered on `stream`: the table that mq_decode_layer reads,
+ * without a host-to-device copy. The reference copies its table once (megakernel_decode.py:129-132). */
+int mq_pack_layer(const LDGLayerWeights* host_layer, LDGLayerWeights* device_layer, hipStream_t stream);
+
 /* Prefill of a whole prompt, then the greedy next token.
  * Replaces `launch_prefill_float` (csrc/megakernel/fused_prefill.cu:601-636) with the
  * same arguments minus the cuBLAS handle (the GEMMs are hand-written MFMA kernels).

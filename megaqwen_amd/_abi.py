@@ -67,6 +67,7 @@ SIGNATURES = {
     # variant, token, out, logits, embed, layers, final norm, lm head, cos, sin, k, v, hidden, normed,
     # num_layers, position, cache_len, max_seq_len, scale, stream
     "mq_decode_variant": [_i, _i, _vp, _vp] + [_vp] * 10 + [_i, _i, _i, _i, _f, _vp],
+    "mq_pack_layer": [_vp, _vp, _vp],
     "mq_decode_layer": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _f, _vp],
     # ids, out, seq_len, embed, layers (host array), final norm, lm head, cos, sin, k, v, 17 scratch,
     # num_layers, max_seq_len, scale, stream

@@ -2271,6 +2271,20 @@ extern "C" int mq_decode_layer(const void* hidden_in, void* hidden_out, const LD
   return launch(P, stream);
 }
 
+// One layer's weight pointers from the launch's arguments into device memory (the decode kernel
+// reads its layer table from there): stream-ordered, where a copy from pageable host memory
+// makes the caller wait (16 us a call for 88 bytes, against 4 us for this launch).
+static __global__ void __launch_bounds__(64) pack_layer_kernel(LDGLayerWeights w, LDGLayerWeights* out) {
+  if (threadIdx.x == 0) *out = w;
+}
+
+extern "C" int mq_pack_layer(const LDGLayerWeights* host_layer, LDGLayerWeights* device_layer, hipStream_t stream) {
+  if (!host_layer || !device_layer) return MQ_ERR_ARG;
+  (void)hipGetLastError();  // clear an error left by an unrelated earlier call
+  pack_layer_kernel<<<1, 64, 0, stream>>>(*host_layer, device_layer);
+  return hipGetLastError() == hipSuccess ? MQ_OK : MQ_ERR_HIP;
+}
+
 extern "C" int mq_decode_step_init(MqDecodeStep* step, int token, int position, int capacity, hipStream_t stream) {
   if (!step || token < 0 || token >= VOCAB || position < 0 || position >= MAX_CTX || capacity < 1) return MQ_ERR_ARG;
   int dev = 0;

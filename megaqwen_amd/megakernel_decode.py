@@ -328,7 +328,7 @@ class MegakernelPrefillDecoder(MegakernelDecoder):
             raise RuntimeError("Empty input sequence")
         if n > self.max_prefill_len_:
             raise RuntimeError("Prefill sequence length exceeds maximum")
-        self.input_tokens_[:n].copy_(ids.to(self.input_tokens_.device), non_blocking=False)
+        self.input_tokens_[:n].copy_(ids)  # (one copy, from wherever the ids are)
         st = _abi.lib().launch_prefill_float(
             _ptr(self.input_tokens_), _ptr(self.output_token_), n, _ptr(self.embed_weight_),
             ctypes.addressof(self.h_layer_weights_), _ptr(self.final_norm_weight_), _ptr(self.lm_head_weight_),
@@ -388,7 +388,7 @@ class MegakernelFusedPrefillDecoder(MegakernelPrefillDecoder):
             raise RuntimeError("Empty input sequence")
         if n > self.max_prefill_len_:
             raise RuntimeError("Prefill sequence length exceeds maximum")
-        self.input_tokens_[:n].copy_(ids.to(self.input_tokens_.device), non_blocking=False)
+        self.input_tokens_[:n].copy_(ids)  # (one copy, from wherever the ids are)
         st = _abi.lib().launch_prefill_megakernel(
             _ptr(self.input_tokens_), _ptr(self.output_token_), n, _ptr(self.embed_weight_),
             ctypes.addressof(self.h_layer_weights_), _ptr(self.final_norm_weight_), _ptr(self.lm_head_weight_),
@@ -417,11 +417,17 @@ def decode_layer(hidden_in: torch.Tensor, layer_weights: list, cos_table, sin_ta
     _check_layer_list(layer_weights, 1)
     max_seq = k_cache.shape[-2]
     out = torch.empty_like(hidden_in)
-    d_lw = make_layer_struct_array(layer_weights, 1)
-    st = _abi.lib().mq_decode_layer(_ptr(hidden_in), _ptr(out), _ptr(d_lw), _ptr(cos_table), _ptr(sin_table),
-                                    _ptr(k_cache), _ptr(v_cache), position, max_seq, attn_scale, _stream())
+    stream = torch.cuda.current_stream()
+    lib, sp = _abi.lib(), stream.cuda_stream
+    # the block's pointer table, written by a launch on the same stream (make_layer_struct_array's
+    # copy from host memory would wait for the device: 16 us a call)
+    table = torch.empty(ctypes.sizeof(_abi.LDGLayerWeights), dtype=torch.uint8, device="cuda")
+    host = _abi.LDGLayerWeights(*[t.data_ptr() for t in layer_weights])
+    _abi.check(lib.mq_pack_layer(ctypes.addressof(host), _ptr(table), sp), "mq_pack_layer")
+    st = lib.mq_decode_layer(_ptr(hidden_in), _ptr(out), _ptr(table), _ptr(cos_table), _ptr(sin_table), _ptr(k_cache),
+                             _ptr(v_cache), position, max_seq, attn_scale, sp)
     _abi.check(st, "mq_decode_layer")
-    torch.cuda.current_stream().synchronize()
+    stream.synchronize()
     return out
 
 
