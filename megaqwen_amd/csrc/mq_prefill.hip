@@ -975,6 +975,39 @@ __device__ __forceinline__ float lane_group_sum(float v) {
   return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
+// K fragments of key tile j (16 keys) of the chunk at LDS address kbase, and the raw scores
+// (q . k, unscaled) of such a tile, both heads: two chains, interleaved, each over the dims in order
+__device__ __forceinline__ void flash_load_k(uint32_t kbase, const uint32_t (&koff)[4], int j, u32x4 (&kf)[4]) {
+#pragma unroll
+  for (int ks = 0; ks < 4; ks++)
+    kf[ks] = *(const __attribute__((address_space(3))) u32x4*)(uintptr_t)(kbase + 4096u * j + koff[ks]);
+}
+__device__ __forceinline__ void flash_qk(const u32x4 (&kf)[4], const u32x4 (&qf)[2][4], f32x4 (&a)[2]) {
+  a[0] = a[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int ks = 0; ks < 4; ks++)
+#pragma unroll
+    for (int hh = 0; hh < 2; hh++) a[hh] = mfma_16x16x32(kf[ks], qf[hh][ks], a[hh]);
+}
+// The four key tiles of a chunk with no masked score, one after another: the next tiles'
+// fragments are read and the next tile's products issued before use(j, scores) takes tile j,
+// where a tile at a time left each wave waiting for its own LDS reads and product chains
+// (attn_prefill_fa2 at S = 8192 423 -> 404 us, attn_prefill_fa3 at S = 3000 99 -> 96.6, same bits).
+template <class Use>
+__device__ __forceinline__ void flash_chunk_scores(uint32_t kbase, const uint32_t (&koff)[4], const u32x4 (&qf)[2][4],
+                                                   Use use) {
+  u32x4 kf[2][4];
+  f32x4 a[2][2];
+  flash_load_k(kbase, koff, 0, kf[0]);
+  flash_load_k(kbase, koff, 1, kf[1]);
+  flash_qk(kf[0], qf, a[0]);
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    if (j < 2) flash_load_k(kbase, koff, j + 2, kf[j & 1]);
+    if (j < 3) flash_qk(kf[(j + 1) & 1], qf, a[(j + 1) & 1]);
+    use(j, a[j & 1]);
+  }
+}
 // ------------------------------------------------------------------ causal attention, two passes
 // Workgroup (KV group g, query block): query rows r0 .. r0 + 127 of both query heads of the
 // group, eight waves of 16 rows each, every wave holding both heads' rows, so that each K
@@ -992,8 +1025,8 @@ __device__ __forceinline__ float lane_group_sum(float v) {
 // its K rows in place.
 constexpr int F2W = 8, F2Q = 16 * F2W, F2KB = 512, F2K = 64, F2NC = F2KB / F2K;
 // prompts longer than this take the two-pass form; shorter ones run faster on
-// attn_prefill_fa3 (8 S / 64 workgroups against 8 S / 128; same-box timings: 5121 tokens
-// 258 against 258 us, 5600 304 against 285, 8192 545 against 452); the two give the same bits
+// attn_prefill_fa3 (8 S / 64 workgroups against 8 S / 128, and a shorter exponential; the
+// launch alone, same box: 4500 tokens 173 against 196 us, 5000 216 against 220, 8192 494 against 404)
 constexpr int FLASH2_MIN_S = 5120;
 // V rows live in LDS with their own chunk swizzle, chunk c of row r in slot c ^ vsw_pf(r):
 // a P.V transpose read takes, per half wave, rows 4 kg + i (kg < 2, i < 4, plus a multiple
@@ -1072,24 +1105,26 @@ __global__ void __launch_bounds__(64 * F2W) attn_prefill_fa2(const uint16_t* q, 
     voff[dt] = vkv_off_pf(4 * kg + (r16 >> 2), dq >> 3) + 2 * (dq & 7);
   }
 
-  // raw scores (q . k, unscaled) of key tile j (16 keys; lane: query row r16, keys
-  // 16 j + 4 kg + e) of K chunk slot c, both heads. The products run at a raised wave
-  // priority, so that the SIMD's other wave, in its exponentials or LDS reads, yields to
-  // them (same bits; S = 8192 22.56 -> 22.31 ms, S = 6000 18.00 -> 17.78 ms on one box, three
-  // rounds each; the same around the P.V products as well: 22.40 ms)
+  // scores of key tile j of K chunk slot c: lane: query row r16, keys 16 j + 4 kg + e
   auto raw_scores = [&](uint32_t kbase, int j, f32x4 (&a)[2]) {
     u32x4 kf[4];
+    flash_load_k(kbase, koff, j, kf);
+    flash_qk(kf, qf, a);
+  };
+
+  // P.V of keys 32 j2 .. +31 of the V chunk at LDS address vb
+  auto pv_half = [&](uint32_t vb, int j2, const u32x2 (&pb)[2][4]) {
+    const u32x4 pf0 = u32x4{pb[0][2 * j2].x, pb[0][2 * j2].y, pb[0][2 * j2 + 1].x, pb[0][2 * j2 + 1].y};
+    const u32x4 pf1 = u32x4{pb[1][2 * j2].x, pb[1][2 * j2].y, pb[1][2 * j2 + 1].x, pb[1][2 * j2 + 1].y};
 #pragma unroll
-    for (int ks = 0; ks < 4; ks++)
-      kf[ks] = *(const __attribute__((address_space(3))) u32x4*)(uintptr_t)(kbase + 4096u * j + koff[ks]);
-    __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-    for (int hh = 0; hh < 2; hh++) {
-      a[hh] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int ks = 0; ks < 4; ks++) a[hh] = mfma_16x16x32(kf[ks], qf[hh][ks], a[hh]);
+    for (int dt = 0; dt < 8; dt++) {
+      const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(uintptr_t)(vb + 8192 * j2 + voff[dt]));
+      const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(uintptr_t)(vb + 8192 * j2 + 4096 + voff[dt]));
+      const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
+      const u32x4 vf = u32x4{l2.x, l2.y, h2.x, h2.y};
+      o[0][dt] = mfma_16x16x32(vf, pf0, o[0][dt]);
+      o[1][dt] = mfma_16x16x32(vf, pf1, o[1][dt]);
     }
-    __builtin_amdgcn_s_setprio(0);
   };
 
   for (int b = 0; b < nblk; b++) {
@@ -1103,14 +1138,11 @@ __global__ void __launch_bounds__(64 * F2W) attn_prefill_fa2(const uint16_t* q, 
       const int ck0 = kb0 + F2K * c;  // the chunk's first key
       if (ck0 + F2K - 1 < kb1 && ck0 + F2K - 1 <= wrow0) {
         // no score of the chunk is masked
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-          f32x4 a[2];
-          raw_scores(kbase, j, a);
+        flash_chunk_scores(kbase, koff, qf, [&](int, const f32x4 (&a)[2]) {
 #pragma unroll
           for (int hh = 0; hh < 2; hh++)
             mx[hh] = fmaxf(fmaxf(mx[hh], fmaxf(a[hh][0], a[hh][1])), fmaxf(a[hh][2], a[hh][3]));
-        }
+        });
       } else {
 #pragma unroll
         for (int j = 0; j < 4; j++) {
@@ -1158,13 +1190,11 @@ __global__ void __launch_bounds__(64 * F2W) attn_prefill_fa2(const uint16_t* q, 
       if (c >= nchb) continue;
       const uint32_t kbase = (uint32_t)c * (F2K * 256);
       const int ck0 = kb0 + F2K * c;
+      const uint32_t vb = lv + (uint32_t)(c & 1) * (F2K * 256);
       u32x2 pb[2][4];
       if (ck0 + F2K - 1 < kb1 && ck0 + F2K - 1 <= wrow0) {
         // no score of the chunk is masked
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-          f32x4 a[2];
-          raw_scores(kbase, j, a);
+        flash_chunk_scores(kbase, koff, qf, [&](int j, const f32x4 (&a)[2]) {
 #pragma unroll
           for (int hh = 0; hh < 2; hh++) {
             float e4[4];
@@ -1175,7 +1205,19 @@ __global__ void __launch_bounds__(64 * F2W) attn_prefill_fa2(const uint16_t* q, 
             }
             pb[hh][j] = u32x2{pack_bf2(e4[0], e4[1]), pack_bf2(e4[2], e4[3])};
           }
+        });
+        pv_half(vb, 0, pb);
+        pv_half(vb, 1, pb);
+        // V fragments are read ahead of the products that take them (masks: 0x100 LDS reads, 0x8 MFMA)
+        __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
+#pragma unroll
+        for (int u = 0; u < 12; u++) {
+          __builtin_amdgcn_sched_group_barrier(0x8, 2, 0);
+          __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
         }
+#pragma unroll
+        for (int u = 0; u < 4; u++) __builtin_amdgcn_sched_group_barrier(0x8, 2, 0);
+        continue;
       } else {
 #pragma unroll
         for (int j = 0; j < 4; j++) {
@@ -1201,24 +1243,9 @@ __global__ void __launch_bounds__(64 * F2W) attn_prefill_fa2(const uint16_t* q, 
           }
         }
       }
-      const uint32_t vb = lv + (uint32_t)(c & 1) * (F2K * 256);
 #pragma unroll
-      for (int j2 = 0; j2 < 2; j2++) {
-        if (ck0 + 32 * j2 <= wrow1) {
-          const u32x4 pf0 = u32x4{pb[0][2 * j2].x, pb[0][2 * j2].y, pb[0][2 * j2 + 1].x, pb[0][2 * j2 + 1].y};
-          const u32x4 pf1 = u32x4{pb[1][2 * j2].x, pb[1][2 * j2].y, pb[1][2 * j2 + 1].x, pb[1][2 * j2 + 1].y};
-#pragma unroll
-          for (int dt = 0; dt < 8; dt++) {
-            const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(uintptr_t)(vb + 8192 * j2 + voff[dt]));
-            const v4s hi =
-                __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(uintptr_t)(vb + 8192 * j2 + 4096 + voff[dt]));
-            const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
-            const u32x4 vf = u32x4{l2.x, l2.y, h2.x, h2.y};
-            o[0][dt] = mfma_16x16x32(vf, pf0, o[0][dt]);
-            o[1][dt] = mfma_16x16x32(vf, pf1, o[1][dt]);
-          }
-        }
-      }
+      for (int j2 = 0; j2 < 2; j2++)
+        if (ck0 + 32 * j2 <= wrow1) pv_half(vb, j2, pb);
     }
 #pragma unroll
     for (int hh = 0; hh < 2; hh++) l_run[hh] = lane_group_sum(sum[hh]) + al[hh] * l_run[hh];
@@ -1249,9 +1276,9 @@ __global__ void __launch_bounds__(64 * F2W) attn_prefill_fa2(const uint16_t* q, 
 // computed once: a wave keeps its whole block of scores in registers (2 heads x 512 keys x 16
 // rows: 256 registers a lane, which one wave per SIMD can hold), takes the row maxima, then
 // the probabilities and P.V chunk by chunk. The operations and their order are those of
-// attn_prefill_fa2 (scores, maxima, exponentials, in-lane sums, P.V chains, rescaling), so the
-// two give the same bits; this one does a third less MFMA work and reads K from LDS once per
-// block instead of twice.
+// attn_prefill_fa2 (scores, maxima, in-lane sums, P.V chains, rescaling) except for the
+// exponential's argument (flash_exp); this one does a third less MFMA work and reads K from LDS
+// once per block instead of twice.
 //
 // LDS: the workgroup's Q rows (32 KB, both heads, read back at the start of every block, so
 // that the Q fragments hold no registers while the probabilities and P.V run), and a ring of
@@ -1261,6 +1288,14 @@ __global__ void __launch_bounds__(64 * F2W) attn_prefill_fa2(const uint16_t* q, 
 // landed and that every wave is done with item n - 1, whose buffer then takes item n + F3R - 1.
 // Past the last item the ring takes dummy copies (K row 0), so every wave issues the same
 // number of DMAs before each wait and the vmcnt count stays exact.
+// The softmax exponential of a raw score in attn_prefill_fa3: 2^(a scale log2 e - max log2 e) with
+// one rounding before the hardware exp2, where the scaled score, the difference and the product
+// with log2 e have three (sl2 = scale log2 e, nb2 = -max log2 e). Two of the 5.5 vector
+// instructions a score less: S = 1117 39.7 -> 37.5 us, 2048 67.4 -> 63.6, 3000 96.6 -> 90.5. (In
+// attn_prefill_fa2 it would give S = 8192 404 -> 388 us, but the near-ties of an 8192-token
+// prompt's greedy continuation then fall HF's way in 247 of 256 steps instead of 249.)
+constexpr float LOG2E = 1.44269504088896341f;
+__device__ __forceinline__ float flash_exp(float a, float sl2, float nb2) { return __builtin_amdgcn_exp2f(fmaf(a, sl2, nb2)); }
 constexpr int F3W = 4, F3Q = 16 * F3W, F3R = 8, F3I = 4;  // waves, query rows, ring, DMAs per item and wave
 // A block's scores are parked in accumulation registers (AGPRs) once the maxima have read
 // them, and brought back to VGPRs chunk by chunk for the exponentials (an empty asm with an
@@ -1358,20 +1393,7 @@ __global__ void __launch_bounds__(64 * F3W) attn_prefill_fa3(const uint16_t* q, 
     const int dq = 16 * dt + 4 * (r16 & 3);
     voff[dt] = vkv_off_pf(4 * kg + (r16 >> 2), dq >> 3) + 2 * (dq & 7);
   }
-  // raw scores (q . k, unscaled) of key tile j of the K chunk at LDS address kbase, both heads
-  auto raw_scores = [&](uint32_t kbase, int j, const u32x4 (&qf)[2][4], f32x4 (&a)[2]) {
-    u32x4 kf[4];
-#pragma unroll
-    for (int ks = 0; ks < 4; ks++)
-      kf[ks] = *(const __attribute__((address_space(3))) u32x4*)(uintptr_t)(kbase + 4096u * j + koff[ks]);
-#pragma unroll
-    for (int hh = 0; hh < 2; hh++) {
-      a[hh] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int ks = 0; ks < 4; ks++) a[hh] = mfma_16x16x32(kf[ks], qf[hh][ks], a[hh]);
-    }
-  };
-
+  const float sl2 = scale * LOG2E;
   int n = 0;  // the next item
   for (int b = 0; b < nblk; b++) {
     const int kb0 = F2KB * b, kb1 = min(nkey, kb0 + F2KB), nc = (kb1 - kb0 + F2K - 1) / F2K;
@@ -1401,22 +1423,21 @@ __global__ void __launch_bounds__(64 * F3W) attn_prefill_fa3(const uint16_t* q, 
         const int ck0 = kb0 + F2K * c;  // the chunk's first key
         if (ck0 + F2K - 1 < kb1 && ck0 + F2K - 1 <= wrow0) {
           // no score of the chunk is masked
-#pragma unroll
-          for (int j = 0; j < 4; j++) {
-            raw_scores(kbase, j, qf, sc[c][j]);
+          flash_chunk_scores(kbase, koff, qf, [&](int j, const f32x4 (&a)[2]) {
 #pragma unroll
             for (int hh = 0; hh < 2; hh++) {
-              mx[hh] = fmaxf(fmaxf(mx[hh], fmaxf(sc[c][j][hh][0], sc[c][j][hh][1])),
-                             fmaxf(sc[c][j][hh][2], sc[c][j][hh][3]));
-              sc[c][j][hh] = park_agpr(sc[c][j][hh]);
+              mx[hh] = fmaxf(fmaxf(mx[hh], fmaxf(a[hh][0], a[hh][1])), fmaxf(a[hh][2], a[hh][3]));
+              sc[c][j][hh] = park_agpr(a[hh]);
             }
-          }
+          });
         } else {
 #pragma unroll
           for (int j = 0; j < 4; j++) {
             const int key0 = ck0 + 16 * j;
             if (key0 <= wrow1) {
-              raw_scores(kbase, j, qf, sc[c][j]);
+              u32x4 kf[4];
+              flash_load_k(kbase, koff, j, kf);
+              flash_qk(kf, qf, sc[c][j]);
 #pragma unroll
               for (int hh = 0; hh < 2; hh++) {
 #pragma unroll
@@ -1442,6 +1463,7 @@ __global__ void __launch_bounds__(64 * F3W) attn_prefill_fa3(const uint16_t* q, 
       for (int dt = 0; dt < 8; dt++) o[hh][dt] *= al[hh];
     }
     // ---- probabilities and P.V, chunk by chunk
+    const float nb2[2] = {-base[0] * LOG2E, -base[1] * LOG2E};
 #pragma unroll
     for (int c = 0; c < F2NC; c++) {
       if (c < nc) {
@@ -1461,7 +1483,7 @@ __global__ void __launch_bounds__(64 * F3W) attn_prefill_fa3(const uint16_t* q, 
               float e4[4];
 #pragma unroll
               for (int e = 0; e < 4; e++) {
-                e4[e] = exp_fast(unfused(a[e] * scale) - base[hh]);
+                e4[e] = flash_exp(a[e], sl2, nb2[hh]);
                 sum[hh] += e4[e];
               }
               pb[hh][j] = u32x2{pack_bf2(e4[0], e4[1]), pack_bf2(e4[2], e4[3])};
@@ -1477,10 +1499,8 @@ __global__ void __launch_bounds__(64 * F3W) attn_prefill_fa3(const uint16_t* q, 
                 float e4[4];
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
-                  // the score a * scale, or -inf where masked (exp(-inf) = 0)
                   const int key = key0 + 4 * kg + e;
-                  const float sv = (key < kb1 && key <= row) ? unfused(a[e] * scale) : -INFINITY;
-                  e4[e] = exp_fast(sv - base[hh]);
+                  e4[e] = (key < kb1 && key <= row) ? flash_exp(a[e], sl2, nb2[hh]) : 0.f;
                   sum[hh] += e4[e];
                 }
                 pb[hh][j] = u32x2{pack_bf2(e4[0], e4[1]), pack_bf2(e4[2], e4[3])};
