@@ -188,17 +188,17 @@ __device__ __forceinline__ int tslot(int r, int kc) { return r * 8 + (kc ^ (r & 
 
 template <int EPI, int TM, int TN, int NST, int KS, int WM, int WN, bool WARM>
 __device__ __forceinline__ void gemm_tiles(const KernArgs<EPI>& G, const WarmSet* W) {
-  constexpr int NW = WM * WN, NT = 64 * NW;
+  constexpr int NW = WM * WN;
   constexpr int RB = TM / (16 * WM);      // 16-row blocks per wave
   constexpr int CB = TN / (16 * WN);      // 16-column blocks per wave
   constexpr int HB = TN / 32;             // EPI_SILU: gate (and up) blocks per tile
   constexpr int ACH = TM * 8, BCH = TN * 8;  // chunk slots of the A and B tiles
   constexpr int SCH = ACH + BCH;          // slots per k-step
-  constexpr int NI = KS * SCH / NT;       // DMA instructions per thread and stage
+  constexpr int NB = KS * SCH / 64;       // 64-slot blocks of a stage, one DMA instruction each
+  constexpr int NI = (NB + NW - 1) / NW;  // DMA instructions per wave and stage
   static_assert(RB * 16 * WM == TM && CB * 16 * WN == TN, "waves tile the output");
   static_assert(EPI != EPI_SILU || CB % 2 == 0, "a wave pairs each gate block with its up block");
-  static_assert(ACH % 64 == 0 && BCH % 64 == 0 && (KS * SCH) % NT == 0,
-                "a DMA instruction covers 64 slots of one operand of one k-step");
+  static_assert(ACH % 64 == 0 && BCH % 64 == 0, "a DMA instruction covers 64 slots of one operand of one k-step");
   __shared__ u32x4 sbuf[NST][KS][SCH];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, wm = wv / WN, wn = wv % WN;
   if (WARM && (int)blockIdx.y == W->row) {
@@ -233,13 +233,14 @@ __device__ __forceinline__ void gemm_tiles(const KernArgs<EPI>& G, const WarmSet
     jb[j] = EPI == EPI_SILU ? (j < CB / 2 ? (CB / 2) * wn + j : HB + (CB / 2) * wn + j - CB / 2) : CB * wn + j;
 
   // DMA instruction i of this wave fills the 64 slots 64 b .. 64 b + 63 of a stage,
-  // b = NW i + wv, counted over the stage's KS k-steps
+  // b = NW i + wv, counted over the stage's KS k-steps (where the waves do not divide the
+  // blocks, the last instruction of some waves copies the last block once more: the same bytes)
   const uint16_t* src[NI];
   uint32_t dst[NI];
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)&sbuf[0][0][0];
 #pragma unroll
   for (int i = 0; i < NI; i++) {
-    const int b0 = 64 * (NW * i + wv), q = b0 / SCH, s0 = b0 % SCH, sl = s0 + lane;
+    const int b0 = 64 * min(NW * i + wv, NB - 1), q = b0 / SCH, s0 = b0 % SCH, sl = s0 + lane;
     dst[i] = __builtin_amdgcn_readfirstlane(lds0 + 16u * (uint32_t)b0);  // wave-uniform (M0)
     const uint16_t* p;
     if (s0 < ACH) {
@@ -326,8 +327,8 @@ __device__ __forceinline__ void gemm_tiles(const KernArgs<EPI>& G, const WarmSet
     // the ring and every accumulator is dead before the rows are processed; then each row of
     // both heads is processed as in the one-head epilogue below, term for term (the norm
     // weights and the row's cos/sin loaded once for both heads).
-    constexpr int RPI = 8 * NW, NPASS = TM / RPI;
-    static_assert(2 * TM * HD * 2 <= NST * KS * SCH * 16 && TM % RPI == 0, "both heads' rows fit the ring");
+    constexpr int RPI = 8 * NW, NPASS = (TM + RPI - 1) / RPI;  // rows a pass of the workgroup
+    static_assert(2 * TM * HD * 2 <= NST * KS * SCH * 16, "both heads' rows fit the ring");
     uint16_t* tile = reinterpret_cast<uint16_t*>(&sbuf[0][0][0]);
     auto slot = [](int hh, int r, int d) { return (hh * TM + r) * HD + 8 * ((d >> 3) ^ (r & 15)) + (d & 7); };
     __syncthreads();  // every wave is past its last read of the ring
@@ -355,7 +356,7 @@ __device__ __forceinline__ void gemm_tiles(const KernArgs<EPI>& G, const WarmSet
 #pragma unroll
       for (int it = 0; it < NPASS; it++) {
         const int r = RPI * it + 8 * wv + rr, t = m0 + r;
-        if (t >= G.m) continue;
+        if (t >= G.m || (TM % RPI && r >= TM)) continue;
 #pragma unroll
         for (int hh = 0; hh < 2; hh++) {
           uint16_t* dst = Q.vc + ((size_t)(2 * nt + hh) * Q.max_seq + t) * HD;
@@ -381,6 +382,7 @@ __device__ __forceinline__ void gemm_tiles(const KernArgs<EPI>& G, const WarmSet
 #pragma unroll
     for (int it = 0; it < NPASS; it++) {
       const int r = RPI * it + 8 * wv + rr, t = m0 + r;
+      if (TM % RPI && r >= TM) continue;
       float c1[8], c2[8], s1[8], s2[8];
       bf8(cs[it][0], c1);
       bf8(cs[it][1], c2);
@@ -1677,13 +1679,11 @@ using namespace mq::pf;
 // o_proj / down_proj always split k four ways, so the choice does not change any result.
 // Longer prompts take larger tiles: a launch streams M N K 2 (1 / TM + 1 / TN) operand
 // bytes from L2 into the CUs, and at S = 8192 the 256 x 256 tiles (sixteen waves, a
-// two-step ring) run gate/up at 840-910 TFLOP/s against 650 for 128 x 128 ones. Short
-// prompts keep smaller tiles so that the grid still fills the 256 CUs:
-//   q/k/v (whole-head tiles, QK-norm/RoPE/K-V-append epilogue): 64 x 128 on 2 x 4 waves;
-//     from S = 1024 128 x 128 on 4 x 2; from 2048 256 x 128 on 4 x 2 with a three-step ring;
-//   gate/up: 128 x 128 on 4 x 4 waves; from S = 1024 128 x 256; from 2048 256 x 256;
-//   o_proj, down_proj (k split four ways into fp32 partials): 128 x 64 on 4 x 2 waves;
-//     from S = 1024 128 x 256 on 2 x 4; from 4096 256 x 256 on 4 x 4.
+// two-step ring) run gate/up at 840-910 TFLOP/s against 650 for 128 x 128 ones. What is lost is
+// mostly a last round of workgroups that leaves CUs idle (144 of 256 for q/k/v at S = 1117 on
+// 128-row tiles), so from 513 (q/k/v) and 641 tokens (gate/up) the row tile is the one whose
+// rounds cost least (row_tile). Whole prefill, same box, before -> now, ms: S = 1117 3.668 -> 3.538,
+// 1300 4.204 -> 3.891, 2500 6.545 -> 6.226, 3000 7.817 -> 7.085, 3500 8.542 -> 8.057, 6000 16.94 -> 16.18.
 constexpr int RES_SPLIT = 4;
 
 // one launch of gemm_nt over a [m, sum of the segments' widths] output, k split `split` ways
@@ -1719,76 +1719,74 @@ void gemm(GemmArgs g, int ntiles, hipStream_t stream, int split = 1, int xg = 0,
     gemm_nt<EPI, TM, TN, NST, KS, WM, WN><<<dim3(ntiles, ny, split), 64 * WM * WN, 0, stream>>>(ka);
   }
 }
+// The row tile of a product of nx workgroups a row tile: of the tiles a shape can take, the one
+// whose rounds of 256 workgroups cost least, `us` a round (one round of that tile, measured; the
+// rounds of a launch follow one another closely enough that two cost about twice one).
+struct RowTile {
+  int tm;
+  float us;
+};
+template <int N>
+static int row_tile(const RowTile (&tiles)[N], int m, int nx) {
+  int best = tiles[0].tm;
+  float cost = INFINITY;
+  for (const RowTile& t : tiles) {
+    const float c = t.us * (float)((nx * ((m + t.tm - 1) / t.tm) + NUM_CUS - 1) / NUM_CUS);
+    if (c < cost) {
+      cost = c;
+      best = t.tm;
+    }
+  }
+  return best;
+}
 static void gemm_qkv(GemmArgs g, hipStream_t stream) {
-  // Long prompts: two heads a tile on sixteen waves (256 x 256, two stages; the epilogue stages
-  // both heads through the ring as bf16), blockIdx order, the same bits as the one-head
-  // 256 x 128 tiles. A two-head tile takes about 1.7 times as long as a one-head tile and there
-  // are half as many, so it is used where its rounds of 256 workgroups, ceil(16 ny / 256), cost
-  // less than the one-head tiles' ceil(32 ny / 256) (ny row tiles). Same box, the q/k/v launch
-  // alone: S = 2600 49.9 -> 40.2 us, 3072 51.9 -> 41.7, 4096 55.0 -> 44.8, 6400 98.8 -> 76.5,
-  // 7168 101.1 -> 80.1, 8192 98.1 -> 82.3; where the model says no: 2048 28.7 -> 39.0, 5000
-  // 74.4 -> 74.0, and the whole S = 6000 prefill 16.58 -> 16.68 ms.
-  const int ny = (g.m + 255) / 256;
-  if (g.m >= 2048 && 17 * ((ny + 15) / 16) < 10 * ((ny + 7) / 8)) {
-    g.seg[0].ntiles = QS / (2 * HD);
-    g.seg[1].ntiles = g.seg[2].ntiles = KVS / (2 * HD);
-    gemm<EPI_QKN, 256, 2 * HD, 2, 1, 4, 4>(g, (QS + 2 * KVS) / (2 * HD), stream);
+  if (g.m <= 512) {
+    // one head a tile, 64 x 128: half the workgroups of 256 columns would leave CUs idle (S = 512
+    // 11.3 us against 16.6 for the two-head tiles)
+    g.seg[0].ntiles = QS / HD;
+    g.seg[1].ntiles = g.seg[2].ntiles = KVS / HD;
+    gemm<EPI_QKN, 64, HD, 4, 1, 2, 4>(g, (QS + 2 * KVS) / HD, stream);
     return;
   }
-  if (g.m > 512 && g.m < 1024) {
-    // 513..1023 tokens: two heads a tile on 64 x 256 tiles (eight waves, four stages), one round
-    // of at most 256 workgroups where the one-head 64 x 128 tiles need two; same bits, the
-    // launch alone, same box: S = 640 19.0 -> 17.1 us, 768 19.6 -> 17.4, 1000 21.2 -> 19.1
-    // (up to 512 tokens the one-head tiles are faster: 11.3 against 16.6 us at S = 512)
-    g.seg[0].ntiles = QS / (2 * HD);
-    g.seg[1].ntiles = g.seg[2].ntiles = KVS / (2 * HD);
-    gemm<EPI_QKN, 64, 2 * HD, 4, 1, 2, 4>(g, (QS + 2 * KVS) / (2 * HD), stream);
-    return;
+  // two heads a tile (both heads' outputs go through the ring as bf16, so nothing spills), 16
+  // column tiles, and the row tile that fills the rounds of 256 workgroups best. The launch
+  // alone with one tile for each range before (64, 128 and 256 rows) -> now, same box, same bits:
+  // S = 1117 22.1 -> 19.6 us, 1300 22.4 -> 20.6, 2500 38.0 -> 31.7, 3000 38.3 -> 33.9
+  constexpr int NX = (QS + 2 * KVS) / (2 * HD);
+  constexpr RowTile TILES[] = {{64, 17.f}, {96, 20.f}, {128, 23.5f}, {160, 31.f}, {192, 33.5f}, {224, 38.f}, {256, 40.f}};
+  g.seg[0].ntiles = QS / (2 * HD);
+  g.seg[1].ntiles = g.seg[2].ntiles = KVS / (2 * HD);
+  switch (row_tile(TILES, g.m, NX)) {
+    case 64: gemm<EPI_QKN, 64, 2 * HD, 4, 1, 2, 4>(g, NX, stream); break;
+    case 96: gemm<EPI_QKN, 96, 2 * HD, 3, 1, 2, 8>(g, NX, stream); break;
+    case 128: gemm<EPI_QKN, 128, 2 * HD, 3, 1, 4, 4>(g, NX, stream); break;
+    case 160: gemm<EPI_QKN, 160, 2 * HD, 2, 1, 2, 8>(g, NX, stream); break;
+    case 192: gemm<EPI_QKN, 192, 2 * HD, 2, 1, 4, 4>(g, NX, stream); break;
+    case 224: gemm<EPI_QKN, 224, 2 * HD, 2, 1, 2, 8>(g, NX, stream); break;
+    default: gemm<EPI_QKN, 256, 2 * HD, 2, 1, 4, 4>(g, NX, stream); break;
   }
-  if (g.m > 1024 && g.m < 2048) {
-    // 1025..2047 tokens: two heads a tile on 128 x 256 tiles (sixteen waves, three stages), one
-    // round of at most 256 workgroups where the one-head 128 x 128 tiles need two (the same
-    // rounds argument as above); same bits, the launch alone, same box: S = 1100 30.6 -> 23.5
-    // us, 1536 31.6 -> 24.4, 2047 33.7 -> 27.2 (at 1024 both take one round)
-    g.seg[0].ntiles = QS / (2 * HD);
-    g.seg[1].ntiles = g.seg[2].ntiles = KVS / (2 * HD);
-    gemm<EPI_QKN, 128, 2 * HD, 3, 1, 4, 4>(g, (QS + 2 * KVS) / (2 * HD), stream);
-    return;
-  }
-  g.seg[0].ntiles = QS / HD;
-  g.seg[1].ntiles = g.seg[2].ntiles = KVS / HD;
-  const int nt = (QS + 2 * KVS) / HD;
-  // long prompts: an XCD takes an eighth of the row tiles and every head, 4 row tiles by 8
-  // heads at a time, so each A row tile is fetched from HBM by one XCD (S = 8192: 107.5 ->
-  // 99.3 us against blockIdx order, same-box medians)
-  if (g.m >= 2048) gemm<EPI_QKN, 256, HD, 3, 1, 4, 2>(g, nt, stream, 1, 1, 4);
-  else if (g.m >= 1024) gemm<EPI_QKN, 128, HD, 4, 1, 4, 2>(g, nt, stream);
-  else gemm<EPI_QKN, 64, HD, 4, 1, 2, 4>(g, nt, stream);
 }
 // warm: the warm-up set of a prompt of at most WARM_MAX_S tokens, or null
 static void gemm_gate_up(GemmArgs g, hipStream_t stream, const WarmSet* warm = nullptr) {
   static_assert(WARM_MAX_S <= 512, "the warm-up set's column tiles are those of the shapes up to 512 tokens");
-  // 2049..3584 tokens: 128 x 256 tiles, twice the workgroups of the 256 x 256 tiles, each
-  // taking about 0.6 of the time; they fill the last round of 256 workgroups better there
-  // (same bits; the launch alone, same box: S = 3072 67.9 -> 61.1 us; at 2048, 5000, 6000
-  // and 7000 the 256 x 256 tiles are as fast or faster, and at 4096 the launch alone gains
-  // (72.0 -> 66.9) but the whole prefill loses, 9.99 -> 10.18 ms)
-  if (g.m > 2048 && g.m <= 3584) {
-    g.seg[0].ntiles = I / 128;
-    gemm<EPI_SILU, 128, 256, 3, 1, 4, 4>(g, I / 128, stream);
-  } else if (g.m > 1408) {
-    // (from 1409 tokens the 128 x 256 tiles need more than one round of 256 workgroups; the
-    // 256 x 256 tiles: S = 1536 38.2 -> 34.5 us, 2047 40.8 -> 38.8; at 1100 22.2 -> 34.5)
-    g.seg[0].ntiles = I / 128;
-    gemm<EPI_SILU, 256, 256, 2, 1, 4, 4>(g, I / 128, stream);  // (the XCD order measured no gain here)
-  } else if (g.m >= 1024) {
-    g.seg[0].ntiles = I / 128;
-    gemm<EPI_SILU, 128, 256, 3, 1, 4, 4>(g, I / 128, stream);
-  } else if (g.m > 640) {
-    // (641..1023 tokens: the 128 x 128 tiles need a second round of 256 workgroups, the
-    // 128 x 256 tiles one; S = 768 24.6 -> 20.5 us, 1000 25.3 -> 21.6; at 640 14.6 -> 19.9)
-    g.seg[0].ntiles = I / 128;
-    gemm<EPI_SILU, 128, 256, 3, 1, 4, 4>(g, I / 128, stream);
+  if (g.m > 640) {
+    // 24 column tiles of 128 units, and the row tile that fills the rounds of 256 workgroups best.
+    // The launch alone with one tile for each range before (128 and 256 rows) -> now, same box,
+    // same bits: S = 800 20.2 -> 18.3 us, 1300 34.0 -> 26.4, 1536 34.0 -> 27.4, 2500 41.6 -> 36.1,
+    // 3000 55.8 -> 44.0, 4000 64.7 -> 58.6 (at 640 the 128 x 128 tiles below stay faster, 14.0
+    // against 17.8). A round of 128-row tiles alone takes 20 us, but in the whole prefill three of
+    // them lose to two of 256 rows (S = 4096 9.80 against 9.61 ms), which 23 reflects
+    constexpr int NX = I / 128;
+    constexpr RowTile TILES[] = {{96, 18.f}, {128, 23.f}, {160, 26.f}, {192, 28.f}, {256, 34.f}, {320, 43.f}};
+    g.seg[0].ntiles = NX;
+    switch (row_tile(TILES, g.m, NX)) {
+      case 96: gemm<EPI_SILU, 96, 256, 3, 1, 2, 8>(g, NX, stream); break;
+      case 128: gemm<EPI_SILU, 128, 256, 3, 1, 4, 4>(g, NX, stream); break;
+      case 160: gemm<EPI_SILU, 160, 256, 2, 1, 2, 8>(g, NX, stream); break;
+      case 192: gemm<EPI_SILU, 192, 256, 2, 1, 4, 4>(g, NX, stream); break;
+      case 256: gemm<EPI_SILU, 256, 256, 2, 1, 4, 4>(g, NX, stream); break;
+      default: gemm<EPI_SILU, 320, 256, 2, 1, 4, 4>(g, NX, stream); break;
+    }
   } else if (g.m > 512) {
     g.seg[0].ntiles = I / 64;
     gemm<EPI_SILU, 128, 128, 3, 1, 4, 4>(g, I / 64, stream, 1, 0, 1, warm);
@@ -1822,9 +1820,14 @@ static void gemm_residual(GemmArgs g, hipStream_t stream) {
   if (g.m > 2048) {
     g.seg[0].ntiles = H / 256;
     gemm<EPI_PART, 256, 256, 2, 1, 4, 4>(g, H / 256, stream, RES_SPLIT);
-  } else if (g.m >= 1024) {
+  } else if (g.m > 1536) {
     g.seg[0].ntiles = H / 256;
     gemm<EPI_PART, 128, 256, 3, 1, 2, 4>(g, H / 256, stream, RES_SPLIT);
+  } else if (g.m >= 1024) {
+    // (96-row tiles on sixteen waves while they take one round; o_proj and down_proj alone: S =
+    // 1117 12.6 -> 11.2 and 16.4 -> 14.1 us, 1300 13.3 -> 12.3 and 17.1 -> 16.0)
+    g.seg[0].ntiles = H / 256;
+    gemm<EPI_PART, 96, 256, 3, 1, 2, 8>(g, H / 256, stream, RES_SPLIT);
   } else if (g.m > 512) {
     // (513..1023 tokens: one round of 256 workgroups on 128 x 128 tiles where 128 x 64 tiles
     // need two; S = 640 15.1 -> 12.5 us, 1000 17.1 -> 15.2)
