@@ -10,6 +10,7 @@
 //   -> resid_norm_rows (partials + residual, post-attention RMSNorm)
 //   -> gemm_nt (gate and up, SiLU(gate) * up epilogue) -> gemm_nt (down_proj, k split)
 //   -> resid_norm_rows (partials + residual, the next layer's input RMSNorm)
+// (from RESADD_MIN_S tokens o_proj and down_proj add the residual themselves, before rmsnorm_rows)
 // then lm_partial (final norm of the last row, tied LM head, per-block argmax) and
 // argmax_final. Prompts of at most 256 tokens run their layers in one launch instead
 // (mq_prefill_short.hip; the same bits). The GEMMs run on v_mfma_f32_16x16x32_bf16 with fp32 accumulation.
@@ -209,13 +210,14 @@ __device__ __forceinline__ void gemm_tiles(const KernArgs<EPI>& G, const WarmSet
   int nt = blockIdx.x, mt = blockIdx.y;  // column tile, row tile
   const int z = blockIdx.z;               // k split
   if (G.xm.xg > 0) {
-    // (the host sets xg only when 8 divides the tile count, xg the column tiles, 8 / xg the
-    // row tiles and xp the row tiles of a band)
+    // (the host sets xg only when xg divides the column tiles, 8 / xg the grid's row tiles and xp
+    // the row tiles of a band; the last band may hold row tiles past the prompt)
     const int nx = G.nx, L = blockIdx.x + nx * blockIdx.y, c = L & 7, s = L >> 3;
     const int cw = nx / G.xm.xg, rh = G.ny / (8 / G.xm.xg), pn = G.xm.xp * cw;
     const int r = s / pn * G.xm.xp + s % pn % G.xm.xp, cc = s % pn / G.xm.xp;
     mt = c / G.xm.xg * rh + r;
     nt = c % G.xm.xg * cw + cc;
+    if (mt * TM >= G.m) return;  // (the whole workgroup, before any barrier)
   }
   int si = 0;
   if constexpr (KernArgs<EPI>::NSEG > 1)
@@ -1688,11 +1690,13 @@ constexpr int RES_SPLIT = 4;
 
 // one launch of gemm_nt over a [m, sum of the segments' widths] output, k split `split` ways
 // The XCD order of a grid of nx column tiles by ny row tiles (XcdMap) with xg column bands and
-// panels of at most xp row tiles (the largest that divides a band), or blockIdx order when
-// the grid does not split into 8 such rectangles.
-static XcdMap xcd_map(int nx, int ny, int xg, int xp) {
+// panels of at most xp row tiles (the largest that divides a band), or blockIdx order when the
+// column tiles do not split into xg bands. ny is rounded up to a multiple of the 8 / xg row
+// bands: the workgroups past the prompt end at once.
+static XcdMap xcd_map(int nx, int& ny, int xg, int xp) {
   const int gy = xg > 0 && xg <= 8 && 8 % xg == 0 ? 8 / xg : 0;
-  if (gy == 0 || xp < 1 || nx % xg || ny % gy) return XcdMap{0, 0};
+  if (gy == 0 || xp < 1 || nx % xg) return XcdMap{0, 0};
+  ny = (ny + gy - 1) / gy * gy;
   const int rh = ny / gy;
   xp = xp < rh ? xp : rh;
   while (rh % xp) xp--;
@@ -1701,7 +1705,7 @@ static XcdMap xcd_map(int nx, int ny, int xg, int xp) {
 template <int EPI, int TM, int TN, int NST, int KS, int WM, int WN>
 void gemm(GemmArgs g, int ntiles, hipStream_t stream, int split = 1, int xg = 0, int xp = 1,
           const WarmSet* warm = nullptr) {
-  const int ny = (g.m + TM - 1) / TM;
+  int ny = (g.m + TM - 1) / TM;
   g.xm = xcd_map(ntiles, ny, xg, xp);
   // a warm-up row only where its workgroups land on CUs no tile uses, eight to an XCD
   // class, in blockIdx order
@@ -1756,14 +1760,16 @@ static void gemm_qkv(GemmArgs g, hipStream_t stream) {
   constexpr RowTile TILES[] = {{64, 17.f}, {96, 20.f}, {128, 23.5f}, {160, 31.f}, {192, 33.5f}, {224, 38.f}, {256, 40.f}};
   g.seg[0].ntiles = QS / (2 * HD);
   g.seg[1].ntiles = g.seg[2].ntiles = KVS / (2 * HD);
+  // the largest take two row bands by four column bands of XCDs (S = 6000 64.8 -> 63.0 us, 8192 83.2 ->
+  // 79.0; smaller ones gain nothing)
   switch (row_tile(TILES, g.m, NX)) {
     case 64: gemm<EPI_QKN, 64, 2 * HD, 4, 1, 2, 4>(g, NX, stream); break;
     case 96: gemm<EPI_QKN, 96, 2 * HD, 3, 1, 2, 8>(g, NX, stream); break;
     case 128: gemm<EPI_QKN, 128, 2 * HD, 3, 1, 4, 4>(g, NX, stream); break;
     case 160: gemm<EPI_QKN, 160, 2 * HD, 2, 1, 2, 8>(g, NX, stream); break;
-    case 192: gemm<EPI_QKN, 192, 2 * HD, 2, 1, 4, 4>(g, NX, stream); break;
-    case 224: gemm<EPI_QKN, 224, 2 * HD, 2, 1, 2, 8>(g, NX, stream); break;
-    default: gemm<EPI_QKN, 256, 2 * HD, 2, 1, 4, 4>(g, NX, stream); break;
+    case 192: gemm<EPI_QKN, 192, 2 * HD, 2, 1, 4, 4>(g, NX, stream, 1, 4, 4); break;
+    case 224: gemm<EPI_QKN, 224, 2 * HD, 2, 1, 2, 8>(g, NX, stream, 1, 4, 4); break;
+    default: gemm<EPI_QKN, 256, 2 * HD, 2, 1, 4, 4>(g, NX, stream, 1, 4, 4); break;
   }
 }
 // warm: the warm-up set of a prompt of at most WARM_MAX_S tokens, or null
@@ -1800,24 +1806,37 @@ static void gemm_gate_up(GemmArgs g, hipStream_t stream, const WarmSet* warm = n
     gemm<EPI_SILU, 128, 96, 3, 1, 4, 1>(g, I / 48, stream, 1, 0, 1, warm);
   }
 }
-// Long prompts: o_proj / down_proj with the residual add in the epilogue (the four k quarters
-// summed in order inside the workgroup: the same bits as the split-four partials and
-// resid_norm_rows), on 256 x 128 tiles; out = h, updated in place
-constexpr int RESADD_MIN_S = 7168;
+// o_proj / down_proj with the residual add in the epilogue (the four k quarters summed in order
+// inside the workgroup: the same bits as the split-four partials and resid_norm_rows); out = h,
+// updated in place. The fp32 partials cost 32 bytes an output written and read again where h costs 4,
+// but they let four times the workgroups run: this form starts where 128-row tiles fill the CUs
+// better than half (tiles of 32 to 64 rows for shorter prompts are even with the partials alone and
+// lose 1-3% in the whole prefill, whose weights and activations are cold). Launch and the norm after
+// it, partials -> this form, us: S = 3000 33.5 -> 24.9 and 40.3 -> 31.9, 6000 62.1 -> 37.8 and 75.9 ->
+// 50.9. Whole prefill, same box, partials -> this form, ms: S = 2049 5.797 -> 5.836, 2200 6.019 -> 6.000, 3000
+// 7.44 -> 7.27, 4300 11.96 -> 11.38, 5400 15.50 -> 14.54, 6000 16.70 -> 15.64, 7000 19.41 -> 18.57.
+constexpr int RESADD_MIN_S = 2177;
 static void gemm_residual_add(GemmArgs g, uint16_t* h, hipStream_t stream) {
+  // 8 column tiles, the row tile by rounds of workgroups (o_proj and down_proj together, us a round;
+  // 96- and 160-row tiles gain nothing over the next larger ones: S = 2500 51 against 50 us, 5000 74
+  // against 73). An XCD takes a quarter of the row tiles and half the column tiles, 4 row tiles at
+  // a time: each A row tile is fetched by two XCDs instead of eight (S = 8192 o_proj 48.8 ->
+  // 40.0 us, down_proj 66.3 -> 54.2; 4000 26.5 -> 24.7 and 36.0 -> 32.1)
+  constexpr int NX = H / 128;
+  constexpr RowTile TILES[] = {{128, 56.f}, {192, 79.f}, {256, 95.f}};
   g.seg[0].out = h;
   g.seg[0].ldo = H;
-  g.seg[0].ntiles = H / 128;
-  // an XCD takes a quarter of the row tiles and half the column tiles, 4 row tiles at a time:
-  // each A row tile is fetched by two XCDs instead of eight (S = 8192, same-box medians:
-  // o_proj 49.3 -> 41.0 us, down_proj 67.8 -> 55.1 us)
-  gemm<EPI_RESADD, 256, 128, 3, 1, 4, 2>(g, H / 128, stream, 1, 2, 4);
+  g.seg[0].ntiles = NX;
+  switch (row_tile(TILES, g.m, NX)) {
+    case 128: gemm<EPI_RESADD, 128, 128, 4, 1, 4, 4>(g, NX, stream, 1, 2, 4); break;
+    case 192: gemm<EPI_RESADD, 192, 128, 3, 1, 4, 4>(g, NX, stream, 1, 2, 4); break;
+    default: gemm<EPI_RESADD, 256, 128, 3, 1, 4, 2>(g, NX, stream, 1, 2, 4); break;
+  }
 }
+// o_proj / down_proj as four k splits of fp32 partials, below RESADD_MIN_S tokens
 static void gemm_residual(GemmArgs g, hipStream_t stream) {
-  // 256 x 256 tiles from 2049 tokens (at most one round of 256 workgroups up to 4096, where
-  // the 128 x 256 tiles need two; same bits, down_proj's shape alone, same box: S = 3072
-  // 37.8 -> 29.9 us; at 2048 the 128 x 256 tiles are faster, 23.1 against 25.1)
   if (g.m > 2048) {
+    // (one round where the 128 x 256 tiles need two)
     g.seg[0].ntiles = H / 256;
     gemm<EPI_PART, 256, 256, 2, 1, 4, 4>(g, H / 256, stream, RES_SPLIT);
   } else if (g.m > 1536) {

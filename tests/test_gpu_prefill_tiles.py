@@ -1,12 +1,14 @@
 """GPU tests of the prefill products' row tiles past 512 tokens.
 
-The row tile of q/k/v and gate/up is chosen by the rounds of workgroups a prompt takes, and every
-tile sums each output in the same order. A row's results depend neither on the tile nor on the
-rows after it, so the first S rows of a longer prompt that runs the same attention kernel are the
-oracle of an S-token prompt, bit for bit. The lengths sit at the edges of the tiles' ranges
-(q/k/v: 64 rows up to 1024 tokens, 96 to 1536, 128 to 2048, 160 to 2560, 192 to 3072, 224 to
-3584, 256 to 4096, 160 to 5120; gate/up: 96 to 960, 128 to 1280, 160 to 1600, 192 to 1920, 256 to
-2560, 320 to 3200, 160 to 3360, 192 to 4032, 256) and one past them, none a multiple of its tile but the first.
+The row tile of q/k/v and gate/up, and past 2176 tokens of o_proj and down_proj, is chosen by the
+rounds of workgroups a prompt takes, and every tile sums each output in the same order. A row's
+results depend neither on the tile nor on the rows after it, so the first S rows of a longer
+prompt that runs the same attention kernel are the oracle of an S-token prompt, bit for bit. The
+lengths sit at the edges of the tiles' ranges and one past them, none a multiple of its tile but
+the first (q/k/v: 64 rows up to 1024 tokens, 96 to 1536, 128 to 2048, 160 to 2560, 192 to 3072,
+224 to 3584, 256 to 4096, 160 to 5120; gate/up: 96 to 960, 128 to 1280, 160 to 1600, 192 to 1920,
+256 to 2560, 320 to 3200, 160 to 3360, 192 to 4032, 256; o_proj and down_proj: fp32 partials to
+2176, then the residual added in the epilogue on 128 rows to 4096, 192 to 6144, 256).
 """
 
 import pytest
@@ -18,8 +20,9 @@ from megaqwen_amd import rope, weights
 pytestmark = pytest.mark.gpu
 
 N_LAYERS = 2
-# attn_prefill serves prompts up to 1024 tokens, attn_prefill_fa3 up to 5120
-LONG = {1024: [513, 641, 959, 961, 1023], 5100: [1025, 1281, 1537, 1601, 1921, 2049, 2561, 3073, 3201, 3361, 3585, 4033, 4097]}
+# attn_prefill serves prompts up to 1024 tokens, attn_prefill_fa3 up to 5120, then attn_prefill_fa2
+LONG = {1024: [513, 641, 959, 961, 1023], 5100: [1025, 1281, 1537, 1601, 1921, 2047, 2049, 2175, 2177, 2561, 3073, 3201, 3361, 3585, 4033, 4097],
+        8200: [5121, 6143, 6145, 8191]}
 
 
 @pytest.fixture(scope="module")
