@@ -5,7 +5,7 @@
 // slots 0..S-1 of every layer are written, and the greedy next token is taken
 // from the last row. After embed_rows and the first layer's rmsnorm_rows, per layer:
 //   gemm_nt (q, k, v in one launch; its epilogue applies QK-norm and RoPE and appends K/V)
-//   -> attn_prefill or, past 1024 tokens, attn_prefill_fa3, past 5120 attn_prefill_fa2 (causal, MFMA)
+//   -> attn_prefill or, past 768 tokens, attn_prefill_fa3, past 6144 attn_prefill_fa2 (causal, MFMA)
 //   -> gemm_nt (o_proj, k split four ways)
 //   -> resid_norm_rows (partials + residual, post-attention RMSNorm)
 //   -> gemm_nt (gate and up, SiLU(gate) * up epilogue) -> gemm_nt (down_proj, k split)
@@ -963,7 +963,10 @@ __global__ void __launch_bounds__(64 * AW) attn_prefill(const uint16_t* q, const
 // of key step j, and V^T is read in the same key order by LDS transpose reads. No score or
 // probability goes through LDS. K and V rows move into LDS in 64-key chunks (16 KB, 1 KB DMA
 // instructions).
-constexpr int FLASH_MIN_S = 1024;  // prompts longer than this take a flash form
+// Prompts longer than this take a flash form (attn_prefill against attn_prefill_fa3: S = 512 14.0
+// and 15.7 us, 700 20.3 and 20.0, 770 26.8 and 21.7, 1024 31.3 and 27.5; whole prefill 700 2.584 and
+// 2.627 ms, 800 2.826 and 2.756).
+constexpr int FLASH_MIN_S = 768;
 
 __device__ __forceinline__ float lane_group_max(float v) {
   const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
@@ -986,22 +989,24 @@ __device__ __forceinline__ void flash_load_k(uint32_t kbase, const uint32_t (&ko
   for (int ks = 0; ks < 4; ks++)
     kf[ks] = *(const __attribute__((address_space(3))) u32x4*)(uintptr_t)(kbase + 4096u * j + koff[ks]);
 }
-__device__ __forceinline__ void flash_qk(const u32x4 (&kf)[4], const u32x4 (&qf)[2][4], f32x4 (&a)[2]) {
-  a[0] = a[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+template <int NH>
+__device__ __forceinline__ void flash_qk(const u32x4 (&kf)[4], const u32x4 (&qf)[NH][4], f32x4 (&a)[NH]) {
+#pragma unroll
+  for (int hh = 0; hh < NH; hh++) a[hh] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int ks = 0; ks < 4; ks++)
 #pragma unroll
-    for (int hh = 0; hh < 2; hh++) a[hh] = mfma_16x16x32(kf[ks], qf[hh][ks], a[hh]);
+    for (int hh = 0; hh < NH; hh++) a[hh] = mfma_16x16x32(kf[ks], qf[hh][ks], a[hh]);
 }
 // The four key tiles of a chunk with no masked score, one after another: the next tiles'
 // fragments are read and the next tile's products issued before use(j, scores) takes tile j,
 // where a tile at a time left each wave waiting for its own LDS reads and product chains
 // (attn_prefill_fa2 at S = 8192 423 -> 404 us, attn_prefill_fa3 at S = 3000 99 -> 96.6, same bits).
-template <class Use>
-__device__ __forceinline__ void flash_chunk_scores(uint32_t kbase, const uint32_t (&koff)[4], const u32x4 (&qf)[2][4],
+template <int NH, class Use>
+__device__ __forceinline__ void flash_chunk_scores(uint32_t kbase, const uint32_t (&koff)[4], const u32x4 (&qf)[NH][4],
                                                    Use use) {
   u32x4 kf[2][4];
-  f32x4 a[2][2];
+  f32x4 a[2][NH];
   flash_load_k(kbase, koff, 0, kf[0]);
   flash_load_k(kbase, koff, 1, kf[1]);
   flash_qk(kf[0], qf, a[0]);
@@ -1021,17 +1026,17 @@ __device__ __forceinline__ void flash_chunk_scores(uint32_t kbase, const uint32_
 // scores and keeps only the row maxima, pass 2 recomputes them, takes the bf16
 // probabilities (held in registers as the B operand of O^T = V^T P^T) and runs that
 // chunk's P.V at once. The sums, the P.V chains and the rescaling happen in the same order
-// as in attn_prefill_fa3, so both give the same bits.
+// as in attn_prefill_fa3 but for the exponential's argument (flash_exp).
 //
 // LDS: the block's 512 K rows (128 KB, resident for both passes) and a two-chunk V ring
 // (32 KB). During pass 2 the next block's K chunk c - 1 is copied into the slot that
 // chunk c - 1 has just left, and V runs one chunk ahead, so pass 1 of the next block finds
 // its K rows in place.
 constexpr int F2W = 8, F2Q = 16 * F2W, F2KB = 512, F2K = 64, F2NC = F2KB / F2K;
-// prompts longer than this take the two-pass form; shorter ones run faster on
-// attn_prefill_fa3 (8 S / 64 workgroups against 8 S / 128, and a shorter exponential; the
-// launch alone, same box: 4500 tokens 173 against 196 us, 5000 216 against 220, 8192 494 against 404)
-constexpr int FLASH2_MIN_S = 5120;
+// prompts longer than this take the two-pass form; shorter ones run faster on attn_prefill_fa3
+// (8 S / 32 workgroups against 8 S / 128, and a shorter exponential; the launch alone, same box,
+// attn_prefill_fa3 against this one: S = 5120 189 and 220 us, 6000 245 and 259, 6500 286 and 281, 8192 443 and 395)
+constexpr int FLASH2_MIN_S = 6144;
 // V rows live in LDS with their own chunk swizzle, chunk c of row r in slot c ^ vsw_pf(r):
 // a P.V transpose read takes, per half wave, rows 4 kg + i (kg < 2, i < 4, plus a multiple
 // of 16) at chunks 2 dt and 2 dt + 1, and vsw_pf = 2 (r % 8) puts those 16 (row, chunk)
@@ -1274,17 +1279,21 @@ __global__ void __launch_bounds__(64 * F2W) attn_prefill_fa2(const uint16_t* q, 
 }
 
 // ------------------------------------------------------------------ causal attention, scores kept
-// Workgroup (KV group g, query block): query rows r0 .. r0 + 63 of both query heads of the
-// group, four waves (one per SIMD) of 16 rows each, every wave holding both heads' rows. Keys
-// run in blocks of 512 with a running maximum, as in attn_prefill_fa2, but each score is
-// computed once: a wave keeps its whole block of scores in registers (2 heads x 512 keys x 16
-// rows: 256 registers a lane, which one wave per SIMD can hold), takes the row maxima, then
-// the probabilities and P.V chunk by chunk. The operations and their order are those of
+// Workgroup (KV group g, query block): query rows r0 .. r0 + 31 of both query heads of the
+// group, four waves of 16 rows of one head. Keys run in blocks of 512 with a running maximum, as
+// in attn_prefill_fa2, but each score is computed once: a wave keeps its whole block of scores
+// in registers (512 keys x 16 rows: 128 a lane), takes the row maxima, then the probabilities
+// and P.V chunk by chunk. With 240 registers and 80 KB of LDS two workgroups share a CU, so a
+// SIMD has two waves whose products, exponentials and LDS reads overlap, and the query blocks
+// are short enough to fill the CUs. Both heads' rows in one wave (64-row blocks, 432 registers,
+// one wave a SIMD) read K and V from LDS half as often and were slower at every length, with the
+// same bits: S = 1024 33.8 -> 26.7 us, 1117 36.8 -> 29.5, 1536 48.5 -> 39.5, 3000 90.2 -> 75.1, 5000
+// 215 -> 179. The operations and their order are those of
 // attn_prefill_fa2 (scores, maxima, in-lane sums, P.V chains, rescaling) except for the
 // exponential's argument (flash_exp); this one does a third less MFMA work and reads K from LDS
 // once per block instead of twice.
 //
-// LDS: the workgroup's Q rows (32 KB, both heads, read back at the start of every block, so
+// LDS: the workgroup's Q rows (16 KB, both heads, read back at the start of every block, so
 // that the Q fragments hold no registers while the probabilities and P.V run), and a ring of
 // F3R chunk buffers (16 KB: 64 K or V rows) through which each block streams its K chunks and
 // then its V chunks ("items"), F3R - 1 items in flight. Before item n a wave
@@ -1300,10 +1309,11 @@ __global__ void __launch_bounds__(64 * F2W) attn_prefill_fa2(const uint16_t* q, 
 // prompt's greedy continuation then fall HF's way in 247 of 256 steps instead of 249.)
 constexpr float LOG2E = 1.44269504088896341f;
 __device__ __forceinline__ float flash_exp(float a, float sl2, float nb2) { return __builtin_amdgcn_exp2f(fmaf(a, sl2, nb2)); }
-constexpr int F3W = 4, F3Q = 16 * F3W, F3R = 8, F3I = 4;  // waves, query rows, ring, DMAs per item and wave
+// waves, heads a wave, query rows, ring, DMAs per item and wave
+constexpr int F3W = 4, F3H = 1, F3Q = 16 * F3W * F3H / 2, F3R = 4, F3I = 4;
 // A block's scores are parked in accumulation registers (AGPRs) once the maxima have read
 // them, and brought back to VGPRs chunk by chunk for the exponentials (an empty asm with an
-// AGPR / VGPR operand: the compiler moves the value there), so that the 256 registers of
+// AGPR / VGPR operand: the compiler moves the value there), so that the 128 registers of
 // scores sit in the AGPR file and the VGPRs keep the operands, accumulators and addresses.
 __device__ __forceinline__ f32x4 park_agpr(f32x4 x) {
   f32x4 r;
@@ -1336,7 +1346,7 @@ __device__ __forceinline__ void fa3_issue(const uint16_t* K, const uint16_t* V, 
   for (int i = 0; i < F3I; i++) dma16(src + (size_t)min(base + drow + 16 * i, kl) * HD + dchk, lds + 4096u * i);
 }
 
-__global__ void __launch_bounds__(64 * F3W) attn_prefill_fa3(const uint16_t* q, const uint16_t* kc, const uint16_t* vc,
+__global__ void __launch_bounds__(64 * F3W, 2) attn_prefill_fa3(const uint16_t* q, const uint16_t* kc, const uint16_t* vc,
                                                               uint16_t* out, int S, int max_seq, float scale) {
   typedef short v4s __attribute__((ext_vector_type(4)));
   typedef __attribute__((address_space(3))) v4s lds_v4s;
@@ -1347,8 +1357,9 @@ __global__ void __launch_bounds__(64 * F3W) attn_prefill_fa3(const uint16_t* q, 
   const int id = blockIdx.x, g = id & 7, nqb = (S + F3Q - 1) / F3Q;  // (the grid: 8 x nqb blocks)
   const int r0 = (nqb - 1 - (id >> 3)) * F3Q;
   const int r16 = lane & 15, kg = lane >> 4;
-  const int row = r0 + 16 * wv + r16;                  // this lane's query row
-  const int wrow0 = r0 + 16 * wv, wrow1 = wrow0 + 15;  // the wave's query rows
+  const int wr = 16 * (wv >> 1), h0 = wv & 1;          // the wave's rows of the block, its head
+  const int row = r0 + wr + r16;                  // this lane's query row
+  const int wrow0 = r0 + wr, wrow1 = wrow0 + 15;  // the wave's query rows
   const int nkey = min(S, r0 + F3Q);
   const int nblk = (nkey + F2KB - 1) / F2KB;
   const int nclast = (nkey - F2KB * (nblk - 1) + F2K - 1) / F2K;  // chunks of the last block
@@ -1367,7 +1378,7 @@ __global__ void __launch_bounds__(64 * F3W) attn_prefill_fa3(const uint16_t* q, 
   auto issue = [&](int n) { fa3_issue(K, V, dchk_k, dchk_v, drow, dl, n, nitems, nblk, nclast, nkey); };
 
   // the Q rows into LDS: [head][row][16-byte chunk slot], chunk c of row r in slot c ^ (r % 16);
-  // instruction i of wave wv moves rows 4 (wv + 4 i) .. +3 of the [2][64] rows, lane -> slot
+  // instruction i of wave wv moves rows 4 (wv + 4 i) .. +3 of the [2][32] rows, lane -> slot
   // lane % 16 of row 4 (wv + 4 i) + lane / 16
   const uint32_t lq = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)&s_q[0][0];
 #pragma unroll
@@ -1376,12 +1387,14 @@ __global__ void __launch_bounds__(64 * F3W) attn_prefill_fa3(const uint16_t* q, 
     dma16(q + (size_t)min(r0 + qr, S - 1) * QS + HD * (2 * g + hh) + 8 * ((lane & 15) ^ (qr & 15)),
           __builtin_amdgcn_readfirstlane(lq + 1024u * (wv + 4 * i)));
   }
-  f32x4 o[2][8];
+  f32x4 o[F3H][8];
 #pragma unroll
-  for (int hh = 0; hh < 2; hh++)
+  for (int hh = 0; hh < F3H; hh++)
 #pragma unroll
     for (int dt = 0; dt < 8; dt++) o[hh][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m_run[2] = {-INFINITY, -INFINITY}, l_run[2] = {0.f, 0.f};
+  float m_run[F3H], l_run[F3H];
+#pragma unroll
+  for (int hh = 0; hh < F3H; hh++) m_run[hh] = -INFINITY, l_run[hh] = 0.f;
   for (int n = 0; n < F3R - 1; n++) issue(n);
   wait_vmem();
   // (the barrier that starts item 0 publishes every wave's Q rows)
@@ -1403,11 +1416,13 @@ __global__ void __launch_bounds__(64 * F3W) attn_prefill_fa3(const uint16_t* q, 
     const int kb0 = F2KB * b, kb1 = min(nkey, kb0 + F2KB), nc = (kb1 - kb0 + F2K - 1) / F2K;
     // ---- the block's scores, kept; the row maxima over the unscaled scores (scale > 0 and
     // rounding is monotonic, so max(a * scale) = max(a) * scale, both rounded)
-    f32x4 sc[F2NC][4][2];
-    float mx[2] = {-INFINITY, -INFINITY};
-    // Q^T (B operand) of both heads: lane (row r16, kg) holds dims 32 ks + 8 kg .. +7 of its
+    f32x4 sc[F2NC][4][F3H];
+    float mx[F3H];
+#pragma unroll
+    for (int hh = 0; hh < F3H; hh++) mx[hh] = -INFINITY;
+    // Q^T (B operand) of the wave's head: lane (row r16, kg) holds dims 32 ks + 8 kg .. +7 of its
     // row (the first item's barrier has published the Q rows; they are never overwritten)
-    u32x4 qf[2][4];
+    u32x4 qf[F3H][4];
 #pragma unroll
     for (int c = 0; c < F2NC; c++) {
       if (c < nc) {
@@ -1418,18 +1433,18 @@ __global__ void __launch_bounds__(64 * F3W) attn_prefill_fa3(const uint16_t* q, 
         n++;
         if (c == 0) {
 #pragma unroll
-          for (int hh = 0; hh < 2; hh++)
+          for (int hh = 0; hh < F3H; hh++)
 #pragma unroll
             for (int ks = 0; ks < 4; ks++)
               qf[hh][ks] = *(const __attribute__((address_space(3))) u32x4*)(uintptr_t)(
-                  lq + 16384u * hh + 256u * 16 * wv + akv_off(r16, 4 * ks + kg));
+                  lq + 256u * F3Q * (h0 + hh) + 256u * wr + akv_off(r16, 4 * ks + kg));
         }
         const int ck0 = kb0 + F2K * c;  // the chunk's first key
         if (ck0 + F2K - 1 < kb1 && ck0 + F2K - 1 <= wrow0) {
           // no score of the chunk is masked
-          flash_chunk_scores(kbase, koff, qf, [&](int j, const f32x4 (&a)[2]) {
+          flash_chunk_scores(kbase, koff, qf, [&](int j, const f32x4 (&a)[F3H]) {
 #pragma unroll
-            for (int hh = 0; hh < 2; hh++) {
+            for (int hh = 0; hh < F3H; hh++) {
               mx[hh] = fmaxf(fmaxf(mx[hh], fmaxf(a[hh][0], a[hh][1])), fmaxf(a[hh][2], a[hh][3]));
               sc[c][j][hh] = park_agpr(a[hh]);
             }
@@ -1443,7 +1458,7 @@ __global__ void __launch_bounds__(64 * F3W) attn_prefill_fa3(const uint16_t* q, 
               flash_load_k(kbase, koff, j, kf);
               flash_qk(kf, qf, sc[c][j]);
 #pragma unroll
-              for (int hh = 0; hh < 2; hh++) {
+              for (int hh = 0; hh < F3H; hh++) {
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
                   const int key = key0 + 4 * kg + e;
@@ -1456,18 +1471,19 @@ __global__ void __launch_bounds__(64 * F3W) attn_prefill_fa3(const uint16_t* q, 
         }
       }
     }
-    float base[2], al[2], sum[2] = {0.f, 0.f};
+    float base[F3H], al[F3H], sum[F3H], nb2[F3H];
 #pragma unroll
-    for (int hh = 0; hh < 2; hh++) {
+    for (int hh = 0; hh < F3H; hh++) {
       const float mn = fmaxf(m_run[hh], lane_group_max(mx[hh]) * scale);
       base[hh] = mn == -INFINITY ? 0.f : mn;
+      sum[hh] = 0.f;
+      nb2[hh] = -base[hh] * LOG2E;
       al[hh] = m_run[hh] == -INFINITY ? 0.f : expf(m_run[hh] - base[hh]);
       m_run[hh] = mn;
 #pragma unroll
       for (int dt = 0; dt < 8; dt++) o[hh][dt] *= al[hh];
     }
     // ---- probabilities and P.V, chunk by chunk
-    const float nb2[2] = {-base[0] * LOG2E, -base[1] * LOG2E};
 #pragma unroll
     for (int c = 0; c < F2NC; c++) {
       if (c < nc) {
@@ -1477,12 +1493,12 @@ __global__ void __launch_bounds__(64 * F3W) attn_prefill_fa3(const uint16_t* q, 
         const uint32_t vb = lr + (uint32_t)(n % F3R) * (F2K * 256);
         n++;
         const int ck0 = kb0 + F2K * c;
-        u32x2 pb[2][4];
+        u32x2 pb[F3H][4];
         if (ck0 + F2K - 1 < kb1 && ck0 + F2K - 1 <= wrow0) {
 #pragma unroll
           for (int j = 0; j < 4; j++)
 #pragma unroll
-            for (int hh = 0; hh < 2; hh++) {
+            for (int hh = 0; hh < F3H; hh++) {
               const f32x4 a = unpark_agpr(sc[c][j][hh]);
               float e4[4];
 #pragma unroll
@@ -1498,7 +1514,7 @@ __global__ void __launch_bounds__(64 * F3W) attn_prefill_fa3(const uint16_t* q, 
             const int key0 = ck0 + 16 * j;
             if (key0 <= wrow1) {
 #pragma unroll
-              for (int hh = 0; hh < 2; hh++) {
+              for (int hh = 0; hh < F3H; hh++) {
                 const f32x4 a = unpark_agpr(sc[c][j][hh]);
                 float e4[4];
 #pragma unroll
@@ -1510,7 +1526,8 @@ __global__ void __launch_bounds__(64 * F3W) attn_prefill_fa3(const uint16_t* q, 
                 pb[hh][j] = u32x2{pack_bf2(e4[0], e4[1]), pack_bf2(e4[2], e4[3])};
               }
             } else {
-              pb[0][j] = pb[1][j] = u32x2{0u, 0u};
+#pragma unroll
+              for (int hh = 0; hh < F3H; hh++) pb[hh][j] = u32x2{0u, 0u};
             }
           }
         }
@@ -1520,8 +1537,10 @@ __global__ void __launch_bounds__(64 * F3W) attn_prefill_fa3(const uint16_t* q, 
           // half's 32 registers of V fragments at a time keeps the kernel within its VGPRs)
           if (j2 == 1) asm volatile("" ::: "memory");
           if (ck0 + 32 * j2 <= wrow1) {
-            const u32x4 pf0 = u32x4{pb[0][2 * j2].x, pb[0][2 * j2].y, pb[0][2 * j2 + 1].x, pb[0][2 * j2 + 1].y};
-            const u32x4 pf1 = u32x4{pb[1][2 * j2].x, pb[1][2 * j2].y, pb[1][2 * j2 + 1].x, pb[1][2 * j2 + 1].y};
+            u32x4 pf[F3H];
+#pragma unroll
+            for (int hh = 0; hh < F3H; hh++)
+              pf[hh] = u32x4{pb[hh][2 * j2].x, pb[hh][2 * j2].y, pb[hh][2 * j2 + 1].x, pb[hh][2 * j2 + 1].y};
 #pragma unroll
             for (int dt = 0; dt < 8; dt++) {
               const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(uintptr_t)(vb + 8192 * j2 + voff[dt]));
@@ -1529,22 +1548,22 @@ __global__ void __launch_bounds__(64 * F3W) attn_prefill_fa3(const uint16_t* q, 
                   __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(uintptr_t)(vb + 8192 * j2 + 4096 + voff[dt]));
               const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
               const u32x4 vf = u32x4{l2.x, l2.y, h2.x, h2.y};
-              o[0][dt] = mfma_16x16x32(vf, pf0, o[0][dt]);
-              o[1][dt] = mfma_16x16x32(vf, pf1, o[1][dt]);
+#pragma unroll
+              for (int hh = 0; hh < F3H; hh++) o[hh][dt] = mfma_16x16x32(vf, pf[hh], o[hh][dt]);
             }
           }
         }
       }
     }
 #pragma unroll
-    for (int hh = 0; hh < 2; hh++) l_run[hh] = lane_group_sum(sum[hh]) + al[hh] * l_run[hh];
+    for (int hh = 0; hh < F3H; hh++) l_run[hh] = lane_group_sum(sum[hh]) + al[hh] * l_run[hh];
   }
   wait_vmem();  // the ring's last (dummy) copies: no DMA may target this LDS after the exit
   if (row < S) {
 #pragma unroll
-    for (int hh = 0; hh < 2; hh++) {
+    for (int hh = 0; hh < F3H; hh++) {
       const float inv = 1.0f / l_run[hh];
-      uint16_t* op = out + (size_t)row * QS + HD * (2 * g + hh) + 4 * kg;
+      uint16_t* op = out + (size_t)row * QS + HD * (2 * g + h0 + hh) + 4 * kg;
 #pragma unroll
       for (int dt = 0; dt < 8; dt++)
         *reinterpret_cast<u32x2*>(op + 16 * dt) =
@@ -1956,7 +1975,7 @@ static int prefill_run(const int* input_token_ids, int* output_token_id, int seq
     gemm_qkv(g, stream);
     chk();
     // long prompts: the two-pass flash form (128 rows of both heads a workgroup), then the
-    // flash form with the scores kept (64 rows); short ones: 32 rows of one head a workgroup,
+    // flash form with the scores kept (32 rows); short ones: 32 rows of one head a workgroup,
     // which fills more CUs (256 workgroups at S = 512)
     if (S > FLASH2_MIN_S)
       attn_prefill_fa2<<<NKV * ((S + F2Q - 1) / F2Q), 64 * F2W, 0, stream>>>(qp, kcl, vcl, att, S, max_seq_len,

@@ -20,9 +20,11 @@ from megaqwen_amd import rope, weights
 pytestmark = pytest.mark.gpu
 
 N_LAYERS = 2
-# attn_prefill serves prompts up to 1024 tokens, attn_prefill_fa3 up to 5120, then attn_prefill_fa2
-LONG = {1024: [513, 641, 959, 961, 1023], 5100: [1025, 1281, 1537, 1601, 1921, 2047, 2049, 2175, 2177, 2561, 3073, 3201, 3361, 3585, 4033, 4097],
-        8200: [5121, 6143, 6145, 8191]}
+# attn_prefill serves prompts up to 768 tokens, attn_prefill_fa3 up to 6144, then attn_prefill_fa2
+LONG = {767: [513, 641],
+        6140: [769, 959, 961, 1023, 1025, 1281, 1537, 1601, 1921, 2047, 2049, 2175, 2177, 2561, 3073, 3201, 3361, 3585,
+               4033, 4097, 5121],
+        8200: [6145, 8191]}
 
 
 @pytest.fixture(scope="module")
