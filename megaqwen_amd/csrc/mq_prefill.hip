@@ -5,7 +5,7 @@
 // slots 0..S-1 of every layer are written, and the greedy next token is taken
 // from the last row. After embed_rows and the first layer's rmsnorm_rows, per layer:
 //   gemm_nt (q, k, v in one launch; its epilogue applies QK-norm and RoPE and appends K/V)
-//   -> attn_prefill or, past 768 tokens, attn_prefill_fa3, past 6144 attn_prefill_fa2 (causal, MFMA)
+//   -> attn_prefill or, past 768 tokens, attn_prefill_fa3, past 5888 attn_prefill_fa2 (causal, MFMA)
 //   -> gemm_nt (o_proj, k split four ways)
 //   -> resid_norm_rows (partials + residual, post-attention RMSNorm)
 //   -> gemm_nt (gate and up, SiLU(gate) * up epilogue) -> gemm_nt (down_proj, k split)
@@ -963,9 +963,11 @@ __global__ void __launch_bounds__(64 * AW) attn_prefill(const uint16_t* q, const
 // of key step j, and V^T is read in the same key order by LDS transpose reads. No score or
 // probability goes through LDS. K and V rows move into LDS in 64-key chunks (16 KB, 1 KB DMA
 // instructions).
-// Prompts longer than this take a flash form (attn_prefill against attn_prefill_fa3: S = 512 14.0
-// and 15.7 us, 700 20.3 and 20.0, 770 26.8 and 21.7, 1024 31.3 and 27.5; whole prefill 700 2.584 and
-// 2.627 ms, 800 2.826 and 2.756).
+// Prompts longer than this take a flash form (whole prefill, same box, attn_prefill against
+// attn_prefill_fa3: S = 700 2.548 and 2.584 ms, 769 2.728 and 2.636, 800 2.770 and 2.688, 1000 3.083
+// and 3.001, 1024 3.181 and 3.118). The two add a row's sum and its P.V products in another order;
+// the attention rows are as far from a 64-bit softmax either way (769 to 1024 tokens, six inputs
+// each: relative 1.81e-3 to 2.01e-3, the two within 1e-8 of each other).
 constexpr int FLASH_MIN_S = 768;
 
 __device__ __forceinline__ float lane_group_max(float v) {
@@ -1026,7 +1028,7 @@ __device__ __forceinline__ void flash_chunk_scores(uint32_t kbase, const uint32_
 // scores and keeps only the row maxima, pass 2 recomputes them, takes the bf16
 // probabilities (held in registers as the B operand of O^T = V^T P^T) and runs that
 // chunk's P.V at once. The sums, the P.V chains and the rescaling happen in the same order
-// as in attn_prefill_fa3 but for the exponential's argument (flash_exp).
+// as in attn_prefill_fa3, so both give the same bits.
 //
 // LDS: the block's 512 K rows (128 KB, resident for both passes) and a two-chunk V ring
 // (32 KB). During pass 2 the next block's K chunk c - 1 is copied into the slot that
@@ -1034,9 +1036,10 @@ __device__ __forceinline__ void flash_chunk_scores(uint32_t kbase, const uint32_
 // its K rows in place.
 constexpr int F2W = 8, F2Q = 16 * F2W, F2KB = 512, F2K = 64, F2NC = F2KB / F2K;
 // prompts longer than this take the two-pass form; shorter ones run faster on attn_prefill_fa3
-// (8 S / 32 workgroups against 8 S / 128, and a shorter exponential; the launch alone, same box,
-// attn_prefill_fa3 against this one: S = 5120 189 and 220 us, 6000 245 and 259, 6500 286 and 281, 8192 443 and 395)
-constexpr int FLASH2_MIN_S = 6144;
+// (8 S / 32 workgroups against 8 S / 128, but four times the K and V traffic from L2; whole prefill,
+// same box, attn_prefill_fa3 against this one: S = 5120 12.43 and 13.12 ms, 5500 14.05 and 14.39, 5800
+// 14.90 and 14.96, 6000 15.37 and 15.27, 6144 15.69 and 15.50). The line is a whole query block.
+constexpr int FLASH2_MIN_S = 46 * F2Q;
 // V rows live in LDS with their own chunk swizzle, chunk c of row r in slot c ^ vsw_pf(r):
 // a P.V transpose read takes, per half wave, rows 4 kg + i (kg < 2, i < 4, plus a multiple
 // of 16) at chunks 2 dt and 2 dt + 1, and vsw_pf = 2 (r % 8) puts those 16 (row, chunk)
@@ -1289,9 +1292,12 @@ __global__ void __launch_bounds__(64 * F2W) attn_prefill_fa2(const uint16_t* q, 
 // one wave a SIMD) read K and V from LDS half as often and were slower at every length, with the
 // same bits: S = 1024 33.8 -> 26.7 us, 1117 36.8 -> 29.5, 1536 48.5 -> 39.5, 3000 90.2 -> 75.1, 5000
 // 215 -> 179. The operations and their order are those of
-// attn_prefill_fa2 (scores, maxima, in-lane sums, P.V chains, rescaling) except for the
-// exponential's argument (flash_exp); this one does a third less MFMA work and reads K from LDS
-// once per block instead of twice.
+// attn_prefill_fa2 (scores, maxima, exponentials, in-lane sums, P.V chains, rescaling), so the
+// two give the same bits; this one does a third less MFMA work and reads K from LDS once per block
+// instead of twice. (The exponent with one rounding, exp2(fma(a, scale log2 e, -max log2 e)),
+// saves two of a score's 5.5 vector instructions and 1.1-1.4% of a prefill of 1117 to 5000 tokens,
+// but its rows were further from a 64-bit softmax for half of the inputs measured, by up to 1.5e-5
+// of the error.)
 //
 // LDS: the workgroup's Q rows (16 KB, both heads, read back at the start of every block, so
 // that the Q fragments hold no registers while the probabilities and P.V run), and a ring of
@@ -1301,14 +1307,6 @@ __global__ void __launch_bounds__(64 * F2W) attn_prefill_fa2(const uint16_t* q, 
 // landed and that every wave is done with item n - 1, whose buffer then takes item n + F3R - 1.
 // Past the last item the ring takes dummy copies (K row 0), so every wave issues the same
 // number of DMAs before each wait and the vmcnt count stays exact.
-// The softmax exponential of a raw score in attn_prefill_fa3: 2^(a scale log2 e - max log2 e) with
-// one rounding before the hardware exp2, where the scaled score, the difference and the product
-// with log2 e have three (sl2 = scale log2 e, nb2 = -max log2 e). Two of the 5.5 vector
-// instructions a score less: S = 1117 39.7 -> 37.5 us, 2048 67.4 -> 63.6, 3000 96.6 -> 90.5. (In
-// attn_prefill_fa2 it would give S = 8192 404 -> 388 us, but the near-ties of an 8192-token
-// prompt's greedy continuation then fall HF's way in 247 of 256 steps instead of 249.)
-constexpr float LOG2E = 1.44269504088896341f;
-__device__ __forceinline__ float flash_exp(float a, float sl2, float nb2) { return __builtin_amdgcn_exp2f(fmaf(a, sl2, nb2)); }
 // waves, heads a wave, query rows, ring, DMAs per item and wave
 constexpr int F3W = 4, F3H = 1, F3Q = 16 * F3W * F3H / 2, F3R = 4, F3I = 4;
 // A block's scores are parked in accumulation registers (AGPRs) once the maxima have read
@@ -1410,7 +1408,6 @@ __global__ void __launch_bounds__(64 * F3W, 2) attn_prefill_fa3(const uint16_t* 
     const int dq = 16 * dt + 4 * (r16 & 3);
     voff[dt] = vkv_off_pf(4 * kg + (r16 >> 2), dq >> 3) + 2 * (dq & 7);
   }
-  const float sl2 = scale * LOG2E;
   int n = 0;  // the next item
   for (int b = 0; b < nblk; b++) {
     const int kb0 = F2KB * b, kb1 = min(nkey, kb0 + F2KB), nc = (kb1 - kb0 + F2K - 1) / F2K;
@@ -1471,13 +1468,12 @@ __global__ void __launch_bounds__(64 * F3W, 2) attn_prefill_fa3(const uint16_t* 
         }
       }
     }
-    float base[F3H], al[F3H], sum[F3H], nb2[F3H];
+    float base[F3H], al[F3H], sum[F3H];
 #pragma unroll
     for (int hh = 0; hh < F3H; hh++) {
       const float mn = fmaxf(m_run[hh], lane_group_max(mx[hh]) * scale);
       base[hh] = mn == -INFINITY ? 0.f : mn;
       sum[hh] = 0.f;
-      nb2[hh] = -base[hh] * LOG2E;
       al[hh] = m_run[hh] == -INFINITY ? 0.f : expf(m_run[hh] - base[hh]);
       m_run[hh] = mn;
 #pragma unroll
@@ -1503,7 +1499,7 @@ __global__ void __launch_bounds__(64 * F3W, 2) attn_prefill_fa3(const uint16_t* 
               float e4[4];
 #pragma unroll
               for (int e = 0; e < 4; e++) {
-                e4[e] = flash_exp(a[e], sl2, nb2[hh]);
+                e4[e] = exp_fast(unfused(a[e] * scale) - base[hh]);
                 sum[hh] += e4[e];
               }
               pb[hh][j] = u32x2{pack_bf2(e4[0], e4[1]), pack_bf2(e4[2], e4[3])};
@@ -1519,8 +1515,10 @@ __global__ void __launch_bounds__(64 * F3W, 2) attn_prefill_fa3(const uint16_t* 
                 float e4[4];
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
+                  // the score a * scale, or -inf where masked (exp(-inf) = 0)
                   const int key = key0 + 4 * kg + e;
-                  e4[e] = (key < kb1 && key <= row) ? flash_exp(a[e], sl2, nb2[hh]) : 0.f;
+                  const float sv = (key < kb1 && key <= row) ? unfused(a[e] * scale) : -INFINITY;
+                  e4[e] = exp_fast(sv - base[hh]);
                   sum[hh] += e4[e];
                 }
                 pb[hh][j] = u32x2{pack_bf2(e4[0], e4[1]), pack_bf2(e4[2], e4[3])};

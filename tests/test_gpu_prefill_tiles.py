@@ -20,7 +20,7 @@ from megaqwen_amd import rope, weights
 pytestmark = pytest.mark.gpu
 
 N_LAYERS = 2
-# attn_prefill serves prompts up to 768 tokens, attn_prefill_fa3 up to 6144, then attn_prefill_fa2
+# attn_prefill serves prompts up to 768 tokens, attn_prefill_fa3 up to 5888, then attn_prefill_fa2
 LONG = {767: [513, 641],
         6140: [769, 959, 961, 1023, 1025, 1281, 1537, 1601, 1921, 2047, 2049, 2175, 2177, 2561, 3073, 3201, 3361, 3585,
                4033, 4097, 5121],
@@ -49,6 +49,21 @@ def test_rows_do_not_depend_on_the_tile(model, long):
     want = _results(dec, long)
     for S in LONG[long]:
         print(f"prefill S={S}", flush=True)
+        dec.prefill_step(ids[:S])
+        for name, got, ref in zip(("k", "v", "attention", "hidden"), _results(dec, S), want):
+            assert torch.equal(got, ref[:, :, :S] if name in "kv" else ref[:S]), (S, name)
+
+
+def test_rows_are_the_same_bits_in_both_flash_forms(model):
+    """attn_prefill_fa3 and attn_prefill_fa2 run the same operations on a score in the same order,
+    so a row's bits do not turn at the length where the one takes over from the other."""
+    dec, ids = model
+    print("prefill S=8200", flush=True)
+    dec.prefill_step(ids[:8200])
+    want = _results(dec, 8200)
+    for S in (769, 1117, 3000, 5888):
+        print(f"prefill S={S}", flush=True)
+        dec.reset()
         dec.prefill_step(ids[:S])
         for name, got, ref in zip(("k", "v", "attention", "hidden"), _results(dec, S), want):
             assert torch.equal(got, ref[:, :, :S] if name in "kv" else ref[:S]), (S, name)
