@@ -170,6 +170,18 @@ int launch_prefill_float(const int* input_token_ids, int* output_token_id, int s
                          void* block_max_vals, void* block_max_idxs, void* hidden_bf16_out, int num_layers,
                          int max_seq_len, float attn_scale, hipStream_t stream);
 
+/* Test hook: launch_prefill_float for a prompt of at most 256 tokens (MQ_ERR_ARG past them) as it
+ * runs where the launch's workgroups cannot be resident on every XCD at once, for instance because
+ * other launches hold the CUs. The same results. */
+int mq_debug_prefill_any_xcd(const int* input_token_ids, int* output_token_id, int seq_len, const void* embed_weight,
+                             const PrefillLayerWeights* layer_weights, const void* final_norm_weight,
+                             const void* lm_head_weight, const void* cos_table, const void* sin_table, void* k_cache,
+                             void* v_cache, void* hidden_bf16, void* residual, void* normalized, void* q_proj,
+                             void* k_proj, void* v_proj, void* attn_out, void* o_proj_out, void* mlp_norm,
+                             void* gate_out, void* up_out, void* mlp_intermediate, void* down_out, void* final_hidden,
+                             void* block_max_vals, void* block_max_idxs, void* hidden_bf16_out, int num_layers,
+                             int max_seq_len, float attn_scale, hipStream_t stream);
+
 /* Prefill through the reference's fused-prefill launcher name and arguments.
  * Replaces `launch_prefill_megakernel` (csrc/megakernel/fused_prefill_megakernel.cu:938-1016;
  * its Python caller, csrc/megakernel/megakernel_decode.py:911-937). The same MFMA prefill as

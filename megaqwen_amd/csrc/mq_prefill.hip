@@ -1912,7 +1912,7 @@ static int prefill_run(const int* input_token_ids, int* output_token_id, int seq
                        const PrefillLayerWeights* layer_weights, const void* final_norm_weight,
                        const void* lm_head_weight, const void* cos_table, const void* sin_table, void* k_cache,
                        void* v_cache, const PrefillBufs& B, int num_layers, int max_seq_len, float attn_scale,
-                       hipStream_t stream) {
+                       hipStream_t stream, bool any_xcd = false) {
   uint32_t* ws = nullptr;
   const int st = current_workspace(&ws);
   if (st != MQ_OK) return st;
@@ -1953,7 +1953,7 @@ static int prefill_run(const int* input_token_ids, int* output_token_id, int seq
     A.cos_t = bf(cos_table); A.sin_t = bf(sin_table);
     A.sync = reinterpret_cast<uint32_t*>(parts.lo[0]); A.local = reinterpret_cast<uint32_t*>(nrm); A.err = err;
     for (int l = 0; l < num_layers; l++) A.lw[l] = layer_weights[l];
-    const int rc = prefill_short_run(input_token_ids, bf(embed_weight), A, stream);
+    const int rc = prefill_short_run(input_token_ids, bf(embed_weight), A, any_xcd, stream);
     return rc == MQ_OK ? lm_head() : rc;
   }
   embed_rows<<<S, 128, 0, stream>>>(input_token_ids, bf(embed_weight), h, err);
@@ -2041,16 +2041,15 @@ static int prefill_run(const int* input_token_ids, int* output_token_id, int seq
   return lm_head();
 }
 
-extern "C" int launch_prefill_float(const int* input_token_ids, int* output_token_id, int seq_len,
-                                    const void* embed_weight, const PrefillLayerWeights* layer_weights,
-                                    const void* final_norm_weight, const void* lm_head_weight, const void* cos_table,
-                                    const void* sin_table, void* k_cache, void* v_cache, void* hidden_bf16,
-                                    void* residual, void* normalized, void* q_proj, void* k_proj, void* v_proj,
-                                    void* attn_out, void* o_proj_out, void* mlp_norm, void* gate_out, void* up_out,
-                                    void* mlp_intermediate, void* down_out, void* final_hidden, void* block_max_vals,
-                                    void* block_max_idxs, void* hidden_bf16_out, int num_layers, int max_seq_len,
-                                    float attn_scale, hipStream_t stream) {
-  (void)residual; (void)o_proj_out; (void)down_out;
+// launch_prefill_float without its unused arguments; any_xcd: see mq_debug_prefill_any_xcd
+static int prefill_float(bool any_xcd, const int* input_token_ids, int* output_token_id, int seq_len,
+                         const void* embed_weight, const PrefillLayerWeights* layer_weights,
+                         const void* final_norm_weight, const void* lm_head_weight, const void* cos_table,
+                         const void* sin_table, void* k_cache, void* v_cache, void* hidden_bf16, void* normalized,
+                         void* q_proj, void* k_proj, void* v_proj, void* attn_out, void* mlp_norm, void* gate_out,
+                         void* up_out, void* mlp_intermediate, void* final_hidden, void* block_max_vals,
+                         void* block_max_idxs, void* hidden_bf16_out, int num_layers, int max_seq_len, float attn_scale,
+                         hipStream_t stream) {
   if (!prefill_args_ok(input_token_ids, output_token_id, seq_len, embed_weight, layer_weights, final_norm_weight,
                        lm_head_weight, cos_table, sin_table, k_cache, v_cache, num_layers, max_seq_len, attn_scale) ||
       !hidden_bf16 || !normalized || !q_proj || !k_proj || !v_proj || !attn_out || !mlp_norm || !gate_out ||
@@ -2085,7 +2084,40 @@ extern "C" int launch_prefill_float(const int* input_token_ids, int* output_toke
   B.bmi = static_cast<int*>(block_max_idxs);
   return prefill_run(input_token_ids, output_token_id, seq_len, embed_weight, layer_weights, final_norm_weight,
                      lm_head_weight, cos_table, sin_table, k_cache, v_cache, B, num_layers, max_seq_len, attn_scale,
-                     stream);
+                     stream, any_xcd);
+}
+
+extern "C" int launch_prefill_float(const int* input_token_ids, int* output_token_id, int seq_len,
+                                    const void* embed_weight, const PrefillLayerWeights* layer_weights,
+                                    const void* final_norm_weight, const void* lm_head_weight, const void* cos_table,
+                                    const void* sin_table, void* k_cache, void* v_cache, void* hidden_bf16,
+                                    void* residual, void* normalized, void* q_proj, void* k_proj, void* v_proj,
+                                    void* attn_out, void* o_proj_out, void* mlp_norm, void* gate_out, void* up_out,
+                                    void* mlp_intermediate, void* down_out, void* final_hidden, void* block_max_vals,
+                                    void* block_max_idxs, void* hidden_bf16_out, int num_layers, int max_seq_len,
+                                    float attn_scale, hipStream_t stream) {
+  (void)residual; (void)o_proj_out; (void)down_out;
+  return prefill_float(false, input_token_ids, output_token_id, seq_len, embed_weight, layer_weights, final_norm_weight,
+                       lm_head_weight, cos_table, sin_table, k_cache, v_cache, hidden_bf16, normalized, q_proj, k_proj,
+                       v_proj, attn_out, mlp_norm, gate_out, up_out, mlp_intermediate, final_hidden, block_max_vals,
+                       block_max_idxs, hidden_bf16_out, num_layers, max_seq_len, attn_scale, stream);
+}
+
+extern "C" int mq_debug_prefill_any_xcd(const int* input_token_ids, int* output_token_id, int seq_len,
+                                        const void* embed_weight, const PrefillLayerWeights* layer_weights,
+                                        const void* final_norm_weight, const void* lm_head_weight, const void* cos_table,
+                                        const void* sin_table, void* k_cache, void* v_cache, void* hidden_bf16,
+                                        void* residual, void* normalized, void* q_proj, void* k_proj, void* v_proj,
+                                        void* attn_out, void* o_proj_out, void* mlp_norm, void* gate_out, void* up_out,
+                                        void* mlp_intermediate, void* down_out, void* final_hidden, void* block_max_vals,
+                                        void* block_max_idxs, void* hidden_bf16_out, int num_layers, int max_seq_len,
+                                        float attn_scale, hipStream_t stream) {
+  (void)residual; (void)o_proj_out; (void)down_out;
+  if (seq_len > ps::SHORT_MAX_S) return MQ_ERR_ARG;
+  return prefill_float(true, input_token_ids, output_token_id, seq_len, embed_weight, layer_weights, final_norm_weight,
+                       lm_head_weight, cos_table, sin_table, k_cache, v_cache, hidden_bf16, normalized, q_proj, k_proj,
+                       v_proj, attn_out, mlp_norm, gate_out, up_out, mlp_intermediate, final_hidden, block_max_vals,
+                       block_max_idxs, hidden_bf16_out, num_layers, max_seq_len, attn_scale, stream);
 }
 
 // The reference's fused-prefill launcher (csrc/megakernel/fused_prefill_megakernel.cu:938-1016),

@@ -16,6 +16,7 @@ struct ShortArgs {
   int S, num_layers, max_seq;
   int groups;  // tasks a column slice's row blocks are dealt to, set by prefill_short_run
   float scale;
+  uint64_t place_ticks;  // wait for workgroups on every XCD (0: a single list at once), set likewise
   uint16_t *h, *q, *att, *mid;  // [S, 1024], [S, 2048], [S, 2048], [S, 3072] bf16
   uint16_t *kc, *vc;            // caches, [layers][8][max_seq][128]
   const uint16_t *cos_t, *sin_t;
@@ -27,7 +28,8 @@ struct ShortArgs {
 }  // namespace ps
 
 // Embedding rows and every layer of a prompt of at most SHORT_MAX_S tokens: h holds the residual
-// stream after the last layer, the caches the prompt's K and V rows. MQ_OK or MQ_ERR_HIP.
-int prefill_short_run(const int* ids, const uint16_t* embed, const ps::ShortArgs& A, hipStream_t stream);
+// stream after the last layer, the caches the prompt's K and V rows. `any_xcd`: as where the launch's
+// workgroups are not resident on every XCD. MQ_OK or MQ_ERR_HIP.
+int prefill_short_run(const int* ids, const uint16_t* embed, const ps::ShortArgs& A, bool any_xcd, hipStream_t stream);
 
 }  // namespace mq

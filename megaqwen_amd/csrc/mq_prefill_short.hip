@@ -26,14 +26,21 @@
 // the tasks that share weight rows share an L2. Each XCD's tasks form one list, ordered by
 // layer and step; a workgroup takes the next task of its XCD's list with an atomic ticket and
 // finishes it before it takes another. A task waits only for tasks of earlier steps, so the
-// earliest unfinished task is either running or next on its XCD's list: the launch makes
-// progress with two or more workgroups resident on each XCD (one is its relay), whatever else runs, and
-// needs no co-residency of its grid. Polls are bounded all the same.
+// earliest unfinished task is either running or next on its XCD's list. A workgroup keeps its CU
+// until its list is done (128 KB of LDS: one a CU), so this makes progress if every XCD has a
+// workgroup for its list and one for its relay, and only then: where launches overlap, two of them
+// could each hold a whole XCD that the other needs. So no task publishes anything before the
+// launch has seen two of its workgroups on every XCD; they stay to the end. Where it has not seen
+// them after PLACE_TICKS (other launches hold the CUs, or the device shows fewer XCDs), it runs
+// from a single list instead (run_tasks<true>): all XCDs' tasks in the same order, each taken by
+// whatever workgroup comes next, and every hand-over device-wide. The earliest unfinished task is
+// then running or next for any workgroup, so one resident workgroup is enough. Polls are bounded
+// all the same.
 //
 // Hand-over. Activations that cross XCDs are written with device-scope (sc1) stores and read
 // with sc1 loads (no stale word in 2e8 reads, and as fast as L2 reads when many CUs read the
 // same rows: 112 GB/s a CU either way; invalidating the L2 instead costs 15 us); q, K and V stay in
-// their XCD. A task's stores are complete (vmcnt(0)) before its flag, layer + 1, is stored. The
+// their XCD (from a single list they cross XCDs too, and are written and read likewise). A task's stores are complete (vmcnt(0)) before its flag, layer + 1, is stored. The
 // buffers are rewritten every layer; a task that overwrites rows depends, through the flags of
 // those rows, on every task that read them (h: o and down of a row block follow all qkv,
 // respectively gu, tasks of it; q, attention rows and MLP rows likewise).
@@ -63,12 +70,17 @@ constexpr int LDS_BYTES = NW * RING * STAGE;
 // slice's weights: 4 x (4 + 2 + 6 + 4) tasks of the products a layer and XCD
 constexpr int GROUPS = 4;
 constexpr uint32_t POLL_LIMIT = 1u << 24;  // some seconds of polling
+// How long a launch waits for two workgroups on every XCD (100 MHz ticks: 100 us; on an idle
+// device they are there within a few microseconds)
+constexpr uint64_t PLACE_TICKS = 10000;
 
 // Words of `sync` (device scope): per XCD a cache line with its ticket and role counters; the
-// dead word; then, for each step and relay wave, a line with one word per XCD.
+// dead word, the launch's mode and the single list's ticket; then, for each step and relay wave, a
+// line with one word per XCD.
 enum : int { S_ATT = 0, S_O = 1, S_GU = 2, S_DOWN = 3, NSTEP = 4 };
-constexpr int SY_ROLE = 1, SY_DEAD = 16, SY_STEPS = 32 * NXCD, SY_LINE = 16;
+constexpr int SY_ROLE = 1, SY_DEAD = 16, SY_MODE = 32 + 16, SY_ANY = 64 + 16, SY_STEPS = 32 * NXCD, SY_LINE = 16;
 constexpr int SYNC_WORDS = SY_STEPS + NSTEP * NW * SY_LINE;
+enum : uint32_t { MODE_XCD = 1, MODE_ANY = 2 };  // a list per XCD; a single list
 static_assert(SYNC_WORDS <= H, "the sync area fits one row of fp32 partial sums");
 // Words of `local`, one region per XCD that only its own workgroups touch: per step and relay
 // wave the relay's word, then the flags of the XCD's tasks, per row block.
@@ -118,9 +130,10 @@ __device__ __forceinline__ void dma16_at_nt(const uint16_t* base, uint32_t off, 
       : "v"(off), "s"(base), "s"(lds)
       : "memory");
 }
-// data of this XCD's own workgroups: past the CU's L1, served by the XCD's L2
-__device__ __forceinline__ u32x4 ld4_nt(const Buf& b, uint32_t off) {
-  return __builtin_amdgcn_raw_buffer_load_b128(b.r, off, 0, 2);
+// data of this XCD's own workgroups: past the CU's L1, served by the XCD's L2; or (ANY) of any XCD's
+template <bool ANY>
+__device__ __forceinline__ u32x4 ld4_xcd(const Buf& b, uint32_t off) {
+  return __builtin_amdgcn_raw_buffer_load_b128(b.r, off, 0, ANY ? SC1 : 2 /* nt */);
 }
 template <int N>
 __device__ __forceinline__ void wait_vm() {
@@ -270,13 +283,15 @@ __device__ __noinline__ bool give_up(const Buf& sb, uint32_t* err, uint32_t spin
   return true;
 }
 // One wave waits until the words of `lb` at `word` (its own in each lane with `mine`) have reached
-// `want`: words of this XCD, stored plainly and read with non-temporal loads served by its L2.
-// False: given up.
+// `want`: words of this XCD, stored plainly and read with non-temporal loads served by its L2, or
+// (ANY) words of every XCD at device scope. False: given up.
+template <bool ANY>
 __device__ __forceinline__ bool wait_local(const Buf& lb, const Buf& sb, uint32_t* err, int word, bool mine,
                                            uint32_t want) {
   for (uint32_t spins = 1;; spins++) {
-    const uint32_t v = mine ? __builtin_amdgcn_raw_buffer_load_b32(lb.r, 4 * word, 0, 2 /* nt */) : want;
+    const uint32_t v = mine ? __builtin_amdgcn_raw_buffer_load_b32(lb.r, 4 * word, 0, ANY ? SC1 : 2 /* nt */) : want;
     if (__ballot((int)(v - want) < 0) == 0) return true;
+    if (ANY) __builtin_amdgcn_s_sleep(1);
     asm volatile("" ::: "memory");  // (every round loads)
     if ((spins & 1023u) == 0 && give_up(sb, err, spins)) return false;
   }
@@ -290,8 +305,38 @@ __device__ __forceinline__ bool wait_xcds(const Buf& sb, uint32_t* err, int word
     if ((spins & 1023u) == 0 && give_up(sb, err, spins)) return false;
   }
 }
+template <bool ANY>
 __device__ __forceinline__ void store_local(const Buf& lb, int word, uint32_t v) {
-  __builtin_amdgcn_raw_buffer_store_b32(v, lb.r, 4 * word, 0, 0);
+  __builtin_amdgcn_raw_buffer_store_b32(v, lb.r, 4 * word, 0, ANY ? SC1 : 0);
+}
+
+// The launch's mode, settled once: one wave of the first workgroup on each XCD waits until every
+// XCD has two workgroups of the launch, or until `ticks` have passed, and the first of them to
+// know writes the word.
+__device__ __forceinline__ uint32_t settle_mode(const Buf& sb, uint32_t* sync, uint64_t ticks, int lane) {
+  const uint64_t t0 = wall_clock64();
+  for (;;) {
+    const uint32_t roles = sb.ld1(4u * (uint32_t)(32 * (lane & (NXCD - 1)) + SY_ROLE));
+    const bool late = wall_clock64() - t0 >= ticks;
+    if (late || __ballot(roles < 2u) == 0) {
+      uint32_t m = 0u;
+      if (lane == 0 && __hip_atomic_compare_exchange_strong(sync + SY_MODE, &m, late ? MODE_ANY : MODE_XCD,
+                                                            __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                            __HIP_MEMORY_SCOPE_AGENT))
+        m = late ? MODE_ANY : MODE_XCD;
+      return __builtin_amdgcn_readfirstlane(m);
+    }
+    asm volatile("" ::: "memory");  // (every round loads)
+  }
+}
+// The other workgroups' wait for it (0: given up)
+__device__ __forceinline__ uint32_t wait_mode(const Buf& sb, uint32_t* err) {
+  for (uint32_t spins = 1;; spins++) {
+    const uint32_t m = __builtin_amdgcn_readfirstlane(sb.ld1(4u * SY_MODE));
+    if (m != 0u) return m;
+    asm volatile("" ::: "memory");  // (every round loads)
+    if ((spins & 1023u) == 0 && give_up(sb, err, spins)) return 0u;
+  }
 }
 
 // The relay workgroup of an XCD: each wave follows G row blocks through their steps, layer by layer.
@@ -311,11 +356,11 @@ __device__ __forceinline__ void relay(const Buf& sb, const Buf& lb, uint32_t* er
       else if (s == S_O) word = F.o + rb * NO, n = NO * blocks;
       else if (s == S_GU) word = F.gu + rb * NGU, n = NGU * blocks;
       else word = F.down + rb * ND, n = ND * blocks;
-      if (!wait_local(lb, sb, err, word + lane, lane < n, (uint32_t)l)) return;
+      if (!wait_local<false>(lb, sb, err, word + lane, lane < n, (uint32_t)l)) return;
       const int line = F.steps + (s * NW + wv) * SY_LINE;
       if (lane == 0) sb.st1((uint32_t)l, 4u * (uint32_t)line);
       if (!wait_xcds(sb, err, line & ~(SY_LINE - 1), (uint32_t)l, lane)) return;
-      if (lane == 0) store_local(lb, F.relay + s * NW + wv, (uint32_t)l);
+      if (lane == 0) store_local<false>(lb, F.relay + s * NW + wv, (uint32_t)l);
     }
 }
 
@@ -347,68 +392,90 @@ constexpr int EPI_OFF = 96 * 1024;            // epilogue tiles, past every acti
 static_assert(AO_OFF + 16 * HD * 2 <= LDS_BYTES, "attention LDS");
 __device__ __forceinline__ uint32_t v_off(int row, int chunk) { return row * 256 + 16 * (chunk ^ (row & 15)); }
 
-__global__ void __launch_bounds__(NT) prefill_short(ShortArgs P) {
-  __shared__ __align__(16) uint8_t lds[LDS_BYTES];
-  __shared__ float s_l[16];
-  __shared__ uint32_t s_ticket, s_ok;
-  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  uint32_t xcc;
-  asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(xcc));
-  const int g = (int)(xcc & (NXCD - 1));  // this XCD's KV group and column slices
+struct Shared {
+  __align__(16) uint8_t lds[LDS_BYTES];
+  float l[16];
+  uint32_t ticket, ok;
+};
+
+__device__ __forceinline__ uint32_t take(uint32_t* word) {
+  return __hip_atomic_fetch_add(word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// A workgroup's tasks: those of XCD g's list that fall to it, or (ANY) of the single list, whose
+// task t is task t / 8 of XCD t % 8's. False if a wait was given up or, with a list per XCD, if the
+// launch's mode is the other one (nothing has been published then: a workgroup looks before
+// the first task it finishes). From the single list a task is one row block and waits before it
+// loads its weights: with the weights in registers across a wait on eight XCDs' flags the
+// compiler spills (211 registers), and this path is there to finish, not for speed.
+template <bool ANY>
+__device__ __forceinline__ bool run_tasks(const ShortArgs& P, Shared& sm, int g, int wv) {
+  uint8_t* const lds = sm.lds;
+  float* const s_l = sm.l;
   const int S = P.S, nb = (S + 15) / 16;
   // G consecutive row blocks to a relay wave. A task of the four products loads its weights once
   // and takes row blocks rb, rb + nq, ..: the blocks below nq run a layer's steps together, the
   // next nq behind them (consecutive blocks to a task would make the attention of the later
   // blocks, which reads all earlier rows, wait for the last round of every qkv task)
-  const int G = (nb + NW - 1) / NW, nq = P.groups;
-  const Sync F(nb, g);
+  const int G = (nb + NW - 1) / NW, nq = ANY ? nb : P.groups;
+  Sync F(nb, g);
   const Buf sb(P.sync), lb(P.local);
   const int n_qkv = NQKV * nq, n_att = NATT * nb, n_o = NO * nq, n_gu = NGU * nq, n_d = ND * nq;
   const int per_layer = n_qkv + n_att + n_o + n_gu + n_d, total = per_layer * P.num_layers;
   uint8_t* ring = lds + wv * RING * STAGE;
+  uint32_t* const tickets = P.sync + (ANY ? SY_ANY : 32 * g);
+  bool placed = ANY, ok = true;  // placed: the mode has been looked at (wave 0)
 
-  auto take = [&](int word = 0) -> uint32_t {
-    return __hip_atomic_fetch_add(P.sync + 32 * g + word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  };
-  // the XCD's first workgroup is its relay
-  if (threadIdx.x == 0) s_ticket = take(SY_ROLE);
   __syncthreads();
-  if (__builtin_amdgcn_readfirstlane(s_ticket) == 0) {
-    relay(sb, lb, P.err, F, nb, G, P.num_layers, wv, threadIdx.x & 63);
-    return;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) s_ticket = take();
+  if (threadIdx.x == 0) sm.ticket = take(tickets);
   for (;;) {
     // (opaque, so that the tasks' address arithmetic is not hoisted out of this loop into
     // registers that the weights need)
     int tid = threadIdx.x;
     asm volatile("" : "+v"(tid));
+    if (ANY) asm volatile("" : "+s"(wv));  // (likewise)
     const int lane = tid & 63, r16 = lane & 15, kg = lane >> 4, rq = 4 * kg;
     __syncthreads();
-    const uint32_t t = __builtin_amdgcn_readfirstlane(s_ticket);
+    uint32_t t = __builtin_amdgcn_readfirstlane(sm.ticket);
+    if (ANY) {
+      g = (int)(t & (NXCD - 1));
+      t >>= 3;
+      F = Sync(nb, g);
+    }
     if (t >= (uint32_t)total) break;
     const int l = (int)t / per_layer;
     int i = (int)t % per_layer;
     const PrefillLayerWeights& W = P.lw[l];
     const uint32_t done = (uint32_t)l + 1u;  // flag value of this layer's tasks
-    bool ok = true;
     auto bf = [](const void* p) { return static_cast<const uint16_t*>(p); };
     // every wave is done loading weights, and the tasks this one reads from are done
     auto ready = [&](int word, bool mine, uint32_t want) {
       if (wv == 0) {
-        const bool r = wait_local(lb, sb, P.err, word, mine, want);
-        if (lane == 0) s_ok = r;
+        if (!placed) placed = wait_mode(sb, P.err) == MODE_XCD;
+        const bool r = placed && wait_local<ANY>(lb, sb, P.err, word, mine, want);
+        if (lane == 0) sm.ok = r;
       }
       __syncthreads();
-      ok = __builtin_amdgcn_readfirstlane(s_ok) != 0;
+      ok = __builtin_amdgcn_readfirstlane(sm.ok) != 0;
     };
-    auto relayed = [&](int step, int rb, uint32_t want) { ready(F.relay + step * NW + rb / G, (threadIdx.x & 63) == 0, want); };
+    // ... where those are all XCDs' tasks of a step and row block: this XCD's relay word, or (ANY)
+    // the tasks' flags themselves, lane 8 j + x task j of XCD x
+    auto relayed = [&](int step, int rb, uint32_t want) {
+      if constexpr (ANY) {
+        const int ln = lane, j = ln >> 3;
+        const Sync X(nb, ln & (NXCD - 1));
+        const int n = step == S_ATT ? NATT : step == S_O ? NO : step == S_GU ? NGU : ND;
+        const int base = step == S_ATT ? X.att : step == S_O ? X.o : step == S_GU ? X.gu : X.down;
+        ready(base + n * rb + j, j < n, want);
+      } else {
+        ready(F.relay + step * NW + rb / G, (threadIdx.x & 63) == 0, want);
+      }
+    };
     // the stores of the task's row block are complete, then its flag
     auto finish = [&](int flag) {
       wait_vmem();
       __syncthreads();
-      if (threadIdx.x == 0) store_local(lb, flag, done);
+      if (threadIdx.x == 0) store_local<ANY>(lb, flag, done);
     };
 
     if (i < n_qkv) {
@@ -417,6 +484,10 @@ __global__ void __launch_bounds__(NT) prefill_short(ShortArgs P) {
       const uint16_t* wp = j < 2 ? bf(W.q_proj_weight) + (size_t)(2 * g + j) * HD * H
                                  : bf(j == 2 ? W.k_proj_weight : W.v_proj_weight) + (size_t)g * HD * H;
       u32x4 b[16][2];
+      if (ANY) {
+        relayed(S_DOWN, rb0, (uint32_t)l);
+        if (!ok) break;
+      }
       load_weights(b, wp + (size_t)16 * wv * H, H, [](int s) { return 64 * s; }, ring, lane);
       const uint16_t* nw = bf(W.input_layernorm_weight);
       const u32x4 wc[2] = {ldw(nw + 8 * lane), ldw(nw + 512 + 8 * lane)};
@@ -427,12 +498,13 @@ __global__ void __launch_bounds__(NT) prefill_short(ShortArgs P) {
       const size_t kvl = ((size_t)l * NKV + g) * P.max_seq * HD;
       const Buf out(j < 2 ? P.q + (2 * g + j) * HD : (j == 2 ? P.kc : P.vc) + kvl);
 #pragma unroll 1
-      for (int rb = rb0; rb < nb; rb += nq) {
+      for (int rb = rb0; rb < (ANY ? rb0 + 1 : nb); rb += nq) {
         const int tk = 16 * rb + er;
         const size_t ct = (size_t)min(tk, S - 1) * HD + ed;
         const uint32_t c1 = ldw1(P.cos_t + ct), c2 = ldw1(P.cos_t + ct + 64);
         const uint32_t s1 = ldw1(P.sin_t + ct), s2 = ldw1(P.sin_t + ct + 64);
-        relayed(S_DOWN, rb, (uint32_t)l);
+        if (ANY) __syncthreads();  // every wave is done loading weights
+        else relayed(S_DOWN, rb, (uint32_t)l);
         if (!ok) break;
         load_rows<H, 16>(P.h, 16 * rb, S, lds, wv, lane);
         __syncthreads();
@@ -469,10 +541,10 @@ __global__ void __launch_bounds__(NT) prefill_short(ShortArgs P) {
                         rbf(bfhi(n2) * bfhi(c2)) + rbf(bfhi(n1) * bfhi(s2)));
         }
         if (tk < S) {
-          // (read by this XCD alone: plain stores)
+          // (with a list per XCD read by this XCD alone: plain stores)
           const uint32_t o = 2u * (uint32_t)((j < 2 ? QS : HD) * tk + ed);
-          __builtin_amdgcn_raw_buffer_store_b32(o1, out.r, o, 0, 0);
-          __builtin_amdgcn_raw_buffer_store_b32(o2, out.r, o + 128u, 0, 0);
+          __builtin_amdgcn_raw_buffer_store_b32(o1, out.r, o, 0, ANY ? SC1 : 0);
+          __builtin_amdgcn_raw_buffer_store_b32(o2, out.r, o + 128u, 0, ANY ? SC1 : 0);
         }
         finish(F.qkv + NQKV * rb + j);
       }
@@ -492,13 +564,15 @@ __global__ void __launch_bounds__(NT) prefill_short(ShortArgs P) {
       const uint16_t* V = P.vc + kvl;
       for (int n = wv; n < nk32 / 4; n += NW) {
         const int row = 4 * n + (lane >> 4), chunk = (lane & 15) ^ (row & 15);
-        dma16_at_nt(V, 2u * (uint32_t)(min(row, nk - 1) * HD + 8 * chunk),
-                     __builtin_amdgcn_readfirstlane(lds_addr(lds) + V_OFF + 1024u * (uint32_t)n));
+        const uint32_t src = 2u * (uint32_t)(min(row, nk - 1) * HD + 8 * chunk);
+        const uint32_t dst = __builtin_amdgcn_readfirstlane(lds_addr(lds) + V_OFF + 1024u * (uint32_t)n);
+        if (ANY) dma16_at_sc1(V, src, dst);
+        else dma16_at_nt(V, src, dst);
       }
       u32x4 qf[4];
 #pragma unroll
       for (int ks = 0; ks < 4; ks++)
-        qf[ks] = ld4_nt(qbuf, 2u * (uint32_t)(min(r0 + r16, S - 1) * QS + 32 * ks + 8 * kg));
+        qf[ks] = ld4_xcd<ANY>(qbuf, 2u * (uint32_t)(min(r0 + r16, S - 1) * QS + 32 * ks + 8 * kg));
       float* sc = reinterpret_cast<float*>(lds + SC_OFF);
       constexpr int KT = MAXK / (16 * NW);  // key tiles a wave
       u32x4 kf[KT][4];
@@ -508,7 +582,7 @@ __global__ void __launch_bounds__(NT) prefill_short(ShortArgs P) {
         if (k0 < nk)
 #pragma unroll
           for (int ks = 0; ks < 4; ks++)
-            kf[n][ks] = ld4_nt(kbuf, 2u * (uint32_t)(min(k0 + r16, nk - 1) * HD + 32 * ks + 8 * kg));
+            kf[n][ks] = ld4_xcd<ANY>(kbuf, 2u * (uint32_t)(min(k0 + r16, nk - 1) * HD + 32 * ks + 8 * kg));
       }
 #pragma unroll
       for (int n = 0; n < KT; n++) {
@@ -599,14 +673,19 @@ __global__ void __launch_bounds__(NT) prefill_short(ShortArgs P) {
         const int n = O ? i : i - n_o - n_gu, ct = NC * g + n % NC, rb0 = n / NC;
         const int z = wv & 3, cb0 = CB * (wv >> 2);  // k quarter, first column block
         u32x4 b[CB * NK][2];
+        if (ANY) {
+          relayed(O ? S_ATT : S_GU, rb0, done);
+          if (!ok) return;
+        }
         load_weights(b, bf(O ? W.o_proj_weight : W.down_proj_weight) + (size_t)(TC * ct + 16 * cb0) * K + KQ * z, K,
                      [](int s) { return (s / NK) * 16 * K + 64 * (s % NK); }, ring, lane);
         const Buf hb(P.h + TC * ct);
         const int er = tid / (TC / 2), ec = 2 * (tid % (TC / 2));
         const bool mine = tid < 8 * TC;  // two columns a thread
 #pragma unroll 1
-        for (int rb = rb0; rb < nb; rb += nq) {
-          relayed(O ? S_ATT : S_GU, rb, done);
+        for (int rb = rb0; rb < (ANY ? rb0 + 1 : nb); rb += nq) {
+          if (ANY) __syncthreads();
+          else relayed(O ? S_ATT : S_GU, rb, done);
           if (!ok) return;
           // the residual rows (their last writers are done: the qkv or gu tasks of these rows read them)
           const int row = 16 * rb + er;
@@ -646,14 +725,19 @@ __global__ void __launch_bounds__(NT) prefill_short(ShortArgs P) {
       // waves 0..3: gate blocks of 16 units, waves 4..7: their up blocks
       const int ub = wv & 3;
       u32x4 b[16][2];
+      if (ANY) {
+        relayed(S_O, rb0, done);
+        if (!ok) break;
+      }
       load_weights(b, bf(wv < 4 ? W.gate_proj_weight : W.up_proj_weight) + (size_t)(64 * ct + 16 * ub) * H, H,
                    [](int s) { return 64 * s; }, ring, lane);
       const uint16_t* nw = bf(W.post_attn_layernorm_weight);
       const u32x4 wc[2] = {ldw(nw + 8 * lane), ldw(nw + 512 + 8 * lane)};
       const Buf out(P.mid + 64 * ct);
 #pragma unroll 1
-      for (int rb = rb0; rb < nb; rb += nq) {
-        relayed(S_O, rb, done);
+      for (int rb = rb0; rb < (ANY ? rb0 + 1 : nb); rb += nq) {
+        if (ANY) __syncthreads();
+        else relayed(S_O, rb, done);
         if (!ok) break;
         load_rows<H, 16>(P.h, 16 * rb, S, lds, wv, lane);
         __syncthreads();
@@ -678,19 +762,47 @@ __global__ void __launch_bounds__(NT) prefill_short(ShortArgs P) {
       if (!ok) break;
     }
     // (not earlier: a ticket held while its workgroup waits is a task that no one prepares)
-    if (tid == 0) s_ticket = take();
+    if (tid == 0) sm.ticket = take(tickets);
+  }
+  return ok;
+}
+
+__global__ void __launch_bounds__(NT) prefill_short(ShortArgs P) {
+  __shared__ Shared sm;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  uint32_t xcc;
+  asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(xcc));
+  const int g = (int)(xcc & (NXCD - 1));  // this XCD's KV group and column slices
+  const Buf sb(P.sync);
+  // the XCD's first workgroup is its relay
+  if (threadIdx.x == 0) sm.ticket = take(P.sync + 32 * g + SY_ROLE);
+  __syncthreads();
+  const bool first = __builtin_amdgcn_readfirstlane(sm.ticket) == 0;
+  if (!first && run_tasks<false>(P, sm, g, wv)) return;
+  __syncthreads();
+  if (wv == 0) {
+    const uint32_t m = first ? settle_mode(sb, P.sync, P.place_ticks, threadIdx.x & 63) : wait_mode(sb, P.err);
+    if (threadIdx.x == 0) sm.ok = m;
+  }
+  __syncthreads();
+  if (__builtin_amdgcn_readfirstlane(sm.ok) == MODE_ANY) {
+    run_tasks<true>(P, sm, 0, wv);
+  } else if (first) {
+    const int nb = (P.S + 15) / 16;
+    relay(sb, Buf(P.local), P.err, Sync(nb, g), nb, (nb + NW - 1) / NW, P.num_layers, wv, threadIdx.x & 63);
   }
 }
 
 }  // namespace ps
 
-int prefill_short_run(const int* ids, const uint16_t* embed, const ps::ShortArgs& A, hipStream_t stream) {
+int prefill_short_run(const int* ids, const uint16_t* embed, const ps::ShortArgs& A, bool any_xcd, hipStream_t stream) {
   const int nb = (A.S + 15) / 16;
   ps::embed_rows_sync<<<A.S, 128, 0, stream>>>(ids, embed, A.h, A.err, A.sync, ps::SYNC_WORDS, A.local,
                                                ps::NXCD * ps::local_words(nb));
   if (hipGetLastError() != hipSuccess) return MQ_ERR_HIP;
   ps::ShortArgs B = A;
   B.groups = nb < ps::GROUPS ? nb : ps::GROUPS;
+  B.place_ticks = any_xcd ? 0 : ps::PLACE_TICKS;
   ps::prefill_short<<<ps::NWG, ps::NT, 0, stream>>>(B);
   return hipGetLastError() == hipSuccess ? MQ_OK : MQ_ERR_HIP;
 }

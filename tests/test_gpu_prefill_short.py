@@ -10,6 +10,7 @@ both paths with the numpy oracle.
 import pytest
 import torch
 
+from megaqwen_amd import _abi
 from megaqwen_amd import megakernel_decode as MK
 from megaqwen_amd import rope, weights
 
@@ -69,3 +70,19 @@ def test_short_prompts_on_two_streams(models):
         assert int(dec.output_token_.item()) >= 0
         assert torch.equal(dec.k_cache_[:, :, :S], want[0][:, :, :S])
         assert torch.equal(dec.hidden_float_[:S], want[3][:S])
+
+
+@pytest.mark.parametrize("S", [1, 16, 17, 64, 65, 129, 256])
+def test_single_list_gives_the_same_bits(models, S, monkeypatch):
+    """The form for launches whose workgroups cannot be on every XCD at once (forced from the
+    host): tasks from one list, every hand-over device-wide."""
+    (dec, _), ids, want = models
+    monkeypatch.setattr(_abi.lib(), "launch_prefill_float", _abi.lib().mq_debug_prefill_any_xcd)
+    print(f"prefill S={S}", flush=True)
+    for rep in range(2):
+        dec.reset()
+        dec.prefill_step(ids[:S])
+        for name, got, ref in zip(("k", "v", "attention", "hidden"), _results(dec, S), want):
+            ref = ref[:, :, :S] if name in "kv" else ref[:S]
+            assert torch.equal(got, ref), (name, rep)
+        assert not dec.k_cache_[:, :, S:].any() and not dec.v_cache_[:, :, S:].any()
