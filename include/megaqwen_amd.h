@@ -160,7 +160,9 @@ int mq_pack_layer(const LDGLayerWeights* host_layer, LDGLayerWeights* device_lay
  *   hidden_bf16_out [1024]: a copy of final_hidden (the last row after the final norm), as
  *                    the reference copies it (csrc/megakernel/fused_prefill.cu:843-849).
  *   On return (stream-ordered): *output_token_id = argmax of the last row's bf16
- *   logits (lowest index on ties), or -2 if an input id was outside [0, 151936). */
+ *   logits (lowest index on ties), or a negative value -(1 + flags): flag 1 if an input id was
+ *   outside [0, 151936), flag 2 if a wait between the workgroups of a prompt of at most 256
+ *   tokens did not end within about 1 s (the caches are then undefined; nothing needs a reset). */
 int launch_prefill_float(const int* input_token_ids, int* output_token_id, int seq_len, const void* embed_weight,
                          const PrefillLayerWeights* layer_weights, const void* final_norm_weight,
                          const void* lm_head_weight, const void* cos_table, const void* sin_table, void* k_cache,
@@ -170,17 +172,22 @@ int launch_prefill_float(const int* input_token_ids, int* output_token_id, int s
                          void* block_max_vals, void* block_max_idxs, void* hidden_bf16_out, int num_layers,
                          int max_seq_len, float attn_scale, hipStream_t stream);
 
-/* Test hook: launch_prefill_float for a prompt of at most 256 tokens (MQ_ERR_ARG past them) as it
- * runs where the launch's workgroups cannot be resident on every XCD at once, for instance because
- * other launches hold the CUs. The same results. */
-int mq_debug_prefill_any_xcd(const int* input_token_ids, int* output_token_id, int seq_len, const void* embed_weight,
-                             const PrefillLayerWeights* layer_weights, const void* final_norm_weight,
-                             const void* lm_head_weight, const void* cos_table, const void* sin_table, void* k_cache,
-                             void* v_cache, void* hidden_bf16, void* residual, void* normalized, void* q_proj,
-                             void* k_proj, void* v_proj, void* attn_out, void* o_proj_out, void* mlp_norm,
-                             void* gate_out, void* up_out, void* mlp_intermediate, void* down_out, void* final_hidden,
-                             void* block_max_vals, void* block_max_idxs, void* hidden_bf16_out, int num_layers,
-                             int max_seq_len, float attn_scale, hipStream_t stream);
+/* Test hook: launch_prefill_float for a prompt of at most 256 tokens (MQ_ERR_ARG past them) under
+ * conditions that the host cannot bring about otherwise. `flags`:
+ *   MQ_DEBUG_PREFILL_ANY_XCD: as where the launch's workgroups cannot be resident on every XCD at
+ *     once, for instance because other launches hold the CUs (the same results);
+ *   MQ_DEBUG_PREFILL_GAVE_UP: with the launch's give-up word set, as a failed wait would set it
+ *     (waits that do not succeed soon give up; the result is -3). */
+#define MQ_DEBUG_PREFILL_ANY_XCD 1
+#define MQ_DEBUG_PREFILL_GAVE_UP 2
+int mq_debug_prefill(int flags, const int* input_token_ids, int* output_token_id, int seq_len, const void* embed_weight,
+                     const PrefillLayerWeights* layer_weights, const void* final_norm_weight,
+                     const void* lm_head_weight, const void* cos_table, const void* sin_table, void* k_cache,
+                     void* v_cache, void* hidden_bf16, void* residual, void* normalized, void* q_proj, void* k_proj,
+                     void* v_proj, void* attn_out, void* o_proj_out, void* mlp_norm, void* gate_out, void* up_out,
+                     void* mlp_intermediate, void* down_out, void* final_hidden, void* block_max_vals,
+                     void* block_max_idxs, void* hidden_bf16_out, int num_layers, int max_seq_len, float attn_scale,
+                     hipStream_t stream);
 
 /* Prefill through the reference's fused-prefill launcher name and arguments.
  * Replaces `launch_prefill_megakernel` (csrc/megakernel/fused_prefill_megakernel.cu:938-1016;

@@ -1647,7 +1647,10 @@ __global__ void __launch_bounds__(256) lm_partial(const uint16_t* hlast, const u
   }
 }
 
-__global__ void __launch_bounds__(256) argmax_final(const float* bmv, const int* bmi, int* out, uint32_t* err) {
+// `dead` (or null): the word that the prompt's own launch sets when a wait gives up; `err`: the
+// device's word for an id outside the vocabulary
+__global__ void __launch_bounds__(256) argmax_final(const float* bmv, const int* bmi, int* out, uint32_t* err,
+                                                    const uint32_t* dead) {
   __shared__ float s_bv[4];
   __shared__ int s_bi[4];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
@@ -1681,9 +1684,9 @@ __global__ void __launch_bounds__(256) argmax_final(const float* bmv, const int*
         v = s_bv[w];
         i = s_bi[w];
       }
-    const uint32_t e = *err;
+    const uint32_t w = *err, e = w | (dead && *dead ? 2u : 0u);
     *out = e ? -(int)(1u + e) : i;
-    if (e) *err = 0u;
+    if (w) *err = 0u;
   }
 }
 
@@ -1912,7 +1915,7 @@ static int prefill_run(const int* input_token_ids, int* output_token_id, int seq
                        const PrefillLayerWeights* layer_weights, const void* final_norm_weight,
                        const void* lm_head_weight, const void* cos_table, const void* sin_table, void* k_cache,
                        void* v_cache, const PrefillBufs& B, int num_layers, int max_seq_len, float attn_scale,
-                       hipStream_t stream, bool any_xcd = false) {
+                       hipStream_t stream, int debug = 0) {
   uint32_t* ws = nullptr;
   const int st = current_workspace(&ws);
   if (st != MQ_OK) return st;
@@ -1936,11 +1939,11 @@ static int prefill_run(const int* input_token_ids, int* output_token_id, int seq
     if (e != hipSuccess && launch_err == hipSuccess) launch_err = e;
   };
   (void)hipGetLastError();  // clear an error left by an unrelated earlier call
-  auto lm_head = [&]() {
+  auto lm_head = [&](const uint32_t* dead) {
     lm_partial<<<LMB, 256, 0, stream>>>(h + (size_t)(S - 1) * H, bf(final_norm_weight), bf(lm_head_weight),
                                         B.final_bf16, B.final_f32, B.hidden_out, B.prenorm_out, B.bmv, B.bmi);
     chk();
-    argmax_final<<<1, 256, 0, stream>>>(B.bmv, B.bmi, output_token_id, err);
+    argmax_final<<<1, 256, 0, stream>>>(B.bmv, B.bmi, output_token_id, err, dead);
     chk();
     return launch_err == hipSuccess ? MQ_OK : MQ_ERR_HIP;
   };
@@ -1953,8 +1956,8 @@ static int prefill_run(const int* input_token_ids, int* output_token_id, int seq
     A.cos_t = bf(cos_table); A.sin_t = bf(sin_table);
     A.sync = reinterpret_cast<uint32_t*>(parts.lo[0]); A.local = reinterpret_cast<uint32_t*>(nrm); A.err = err;
     for (int l = 0; l < num_layers; l++) A.lw[l] = layer_weights[l];
-    const int rc = prefill_short_run(input_token_ids, bf(embed_weight), A, any_xcd, stream);
-    return rc == MQ_OK ? lm_head() : rc;
+    const int rc = prefill_short_run(input_token_ids, bf(embed_weight), A, debug, stream);
+    return rc == MQ_OK ? lm_head(A.sync + ps::DEAD_WORD) : rc;
   }
   embed_rows<<<S, 128, 0, stream>>>(input_token_ids, bf(embed_weight), h, err);
   chk();
@@ -2038,11 +2041,11 @@ static int prefill_run(const int* input_token_ids, int* output_token_id, int seq
     }
     chk();
   }
-  return lm_head();
+  return lm_head(nullptr);
 }
 
-// launch_prefill_float without its unused arguments; any_xcd: see mq_debug_prefill_any_xcd
-static int prefill_float(bool any_xcd, const int* input_token_ids, int* output_token_id, int seq_len,
+// launch_prefill_float without its unused arguments; debug: MQ_DEBUG_PREFILL_* flags
+static int prefill_float(int debug, const int* input_token_ids, int* output_token_id, int seq_len,
                          const void* embed_weight, const PrefillLayerWeights* layer_weights,
                          const void* final_norm_weight, const void* lm_head_weight, const void* cos_table,
                          const void* sin_table, void* k_cache, void* v_cache, void* hidden_bf16, void* normalized,
@@ -2084,7 +2087,7 @@ static int prefill_float(bool any_xcd, const int* input_token_ids, int* output_t
   B.bmi = static_cast<int*>(block_max_idxs);
   return prefill_run(input_token_ids, output_token_id, seq_len, embed_weight, layer_weights, final_norm_weight,
                      lm_head_weight, cos_table, sin_table, k_cache, v_cache, B, num_layers, max_seq_len, attn_scale,
-                     stream, any_xcd);
+                     stream, debug);
 }
 
 extern "C" int launch_prefill_float(const int* input_token_ids, int* output_token_id, int seq_len,
@@ -2097,24 +2100,24 @@ extern "C" int launch_prefill_float(const int* input_token_ids, int* output_toke
                                     void* block_max_idxs, void* hidden_bf16_out, int num_layers, int max_seq_len,
                                     float attn_scale, hipStream_t stream) {
   (void)residual; (void)o_proj_out; (void)down_out;
-  return prefill_float(false, input_token_ids, output_token_id, seq_len, embed_weight, layer_weights, final_norm_weight,
+  return prefill_float(0, input_token_ids, output_token_id, seq_len, embed_weight, layer_weights, final_norm_weight,
                        lm_head_weight, cos_table, sin_table, k_cache, v_cache, hidden_bf16, normalized, q_proj, k_proj,
                        v_proj, attn_out, mlp_norm, gate_out, up_out, mlp_intermediate, final_hidden, block_max_vals,
                        block_max_idxs, hidden_bf16_out, num_layers, max_seq_len, attn_scale, stream);
 }
 
-extern "C" int mq_debug_prefill_any_xcd(const int* input_token_ids, int* output_token_id, int seq_len,
-                                        const void* embed_weight, const PrefillLayerWeights* layer_weights,
-                                        const void* final_norm_weight, const void* lm_head_weight, const void* cos_table,
-                                        const void* sin_table, void* k_cache, void* v_cache, void* hidden_bf16,
-                                        void* residual, void* normalized, void* q_proj, void* k_proj, void* v_proj,
-                                        void* attn_out, void* o_proj_out, void* mlp_norm, void* gate_out, void* up_out,
-                                        void* mlp_intermediate, void* down_out, void* final_hidden, void* block_max_vals,
-                                        void* block_max_idxs, void* hidden_bf16_out, int num_layers, int max_seq_len,
-                                        float attn_scale, hipStream_t stream) {
+extern "C" int mq_debug_prefill(int flags, const int* input_token_ids, int* output_token_id, int seq_len,
+                                const void* embed_weight, const PrefillLayerWeights* layer_weights,
+                                const void* final_norm_weight, const void* lm_head_weight, const void* cos_table,
+                                const void* sin_table, void* k_cache, void* v_cache, void* hidden_bf16,
+                                void* residual, void* normalized, void* q_proj, void* k_proj, void* v_proj,
+                                void* attn_out, void* o_proj_out, void* mlp_norm, void* gate_out, void* up_out,
+                                void* mlp_intermediate, void* down_out, void* final_hidden, void* block_max_vals,
+                                void* block_max_idxs, void* hidden_bf16_out, int num_layers, int max_seq_len,
+                                float attn_scale, hipStream_t stream) {
   (void)residual; (void)o_proj_out; (void)down_out;
   if (seq_len > ps::SHORT_MAX_S) return MQ_ERR_ARG;
-  return prefill_float(true, input_token_ids, output_token_id, seq_len, embed_weight, layer_weights, final_norm_weight,
+  return prefill_float(flags, input_token_ids, output_token_id, seq_len, embed_weight, layer_weights, final_norm_weight,
                        lm_head_weight, cos_table, sin_table, k_cache, v_cache, hidden_bf16, normalized, q_proj, k_proj,
                        v_proj, attn_out, mlp_norm, gate_out, up_out, mlp_intermediate, final_hidden, block_max_vals,
                        block_max_idxs, hidden_bf16_out, num_layers, max_seq_len, attn_scale, stream);

@@ -11,6 +11,7 @@ namespace mq {
 namespace ps {
 
 constexpr int SHORT_MAX_S = 256;  // longest prompt it takes
+constexpr int DEAD_WORD = 16;     // word of `sync` that is set once a wait of the launch has given up
 
 struct ShortArgs {
   int S, num_layers, max_seq;
@@ -28,8 +29,8 @@ struct ShortArgs {
 }  // namespace ps
 
 // Embedding rows and every layer of a prompt of at most SHORT_MAX_S tokens: h holds the residual
-// stream after the last layer, the caches the prompt's K and V rows. `any_xcd`: as where the launch's
-// workgroups are not resident on every XCD. MQ_OK or MQ_ERR_HIP.
-int prefill_short_run(const int* ids, const uint16_t* embed, const ps::ShortArgs& A, bool any_xcd, hipStream_t stream);
+// stream after the last layer, the caches the prompt's K and V rows. `debug`: MQ_DEBUG_PREFILL_* flags.
+// MQ_OK or MQ_ERR_HIP.
+int prefill_short_run(const int* ids, const uint16_t* embed, const ps::ShortArgs& A, int debug, hipStream_t stream);
 
 }  // namespace mq

@@ -69,7 +69,7 @@ constexpr int LDS_BYTES = NW * RING * STAGE;
 // A column slice's row blocks are dealt to at most this many tasks, each of which loads the
 // slice's weights: 4 x (4 + 2 + 6 + 4) tasks of the products a layer and XCD
 constexpr int GROUPS = 4;
-constexpr uint32_t POLL_LIMIT = 1u << 24;  // some seconds of polling
+constexpr uint32_t POLL_LIMIT = 1u << 21;  // about 1 s of polling
 // How long a launch waits for two workgroups on every XCD (100 MHz ticks: 100 us; on an idle
 // device they are there within a few microseconds)
 constexpr uint64_t PLACE_TICKS = 10000;
@@ -78,7 +78,7 @@ constexpr uint64_t PLACE_TICKS = 10000;
 // dead word, the launch's mode and the single list's ticket; then, for each step and relay wave, a
 // line with one word per XCD.
 enum : int { S_ATT = 0, S_O = 1, S_GU = 2, S_DOWN = 3, NSTEP = 4 };
-constexpr int SY_ROLE = 1, SY_DEAD = 16, SY_MODE = 32 + 16, SY_ANY = 64 + 16, SY_STEPS = 32 * NXCD, SY_LINE = 16;
+constexpr int SY_ROLE = 1, SY_DEAD = DEAD_WORD, SY_MODE = 32 + 16, SY_ANY = 64 + 16, SY_STEPS = 32 * NXCD, SY_LINE = 16;
 constexpr int SYNC_WORDS = SY_STEPS + NSTEP * NW * SY_LINE;
 enum : uint32_t { MODE_XCD = 1, MODE_ANY = 2 };  // a list per XCD; a single list
 static_assert(SYNC_WORDS <= H, "the sync area fits one row of fp32 partial sums");
@@ -273,36 +273,34 @@ __device__ __forceinline__ void norm_rows(uint8_t* lds, const u32x4 (&wc)[2], in
   }
 }
 
-// Polls are bounded: after POLL_LIMIT rounds a wave sets the dead word and the prompt's error
-// word, and every wait gives up.
-__device__ __noinline__ bool give_up(const Buf& sb, uint32_t* err, uint32_t spins) {
+// Polls are bounded: after POLL_LIMIT rounds a wave sets the launch's dead word, every wait gives up,
+// and the launch's result says so (the word is its own: launches that overlap do not share it).
+__device__ __noinline__ bool give_up(const Buf& sb, uint32_t spins) {
   if (sb.ld1(4u * SY_DEAD) != 0) return true;
   if (spins <= POLL_LIMIT) return false;
   sb.st1(1u, 4u * SY_DEAD);
-  if ((threadIdx.x & 63) == 0) __hip_atomic_fetch_or(err, 2u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   return true;
 }
 // One wave waits until the words of `lb` at `word` (its own in each lane with `mine`) have reached
 // `want`: words of this XCD, stored plainly and read with non-temporal loads served by its L2, or
 // (ANY) words of every XCD at device scope. False: given up.
 template <bool ANY>
-__device__ __forceinline__ bool wait_local(const Buf& lb, const Buf& sb, uint32_t* err, int word, bool mine,
-                                           uint32_t want) {
+__device__ __forceinline__ bool wait_local(const Buf& lb, const Buf& sb, int word, bool mine, uint32_t want) {
   for (uint32_t spins = 1;; spins++) {
     const uint32_t v = mine ? __builtin_amdgcn_raw_buffer_load_b32(lb.r, 4 * word, 0, ANY ? SC1 : 2 /* nt */) : want;
     if (__ballot((int)(v - want) < 0) == 0) return true;
     if (ANY) __builtin_amdgcn_s_sleep(1);
     asm volatile("" ::: "memory");  // (every round loads)
-    if ((spins & 1023u) == 0 && give_up(sb, err, spins)) return false;
+    if ((spins & 1023u) == 0 && give_up(sb, spins)) return false;
   }
 }
 // The same for the eight XCDs' words of a line of `sb`
-__device__ __forceinline__ bool wait_xcds(const Buf& sb, uint32_t* err, int word, uint32_t want, int lane) {
+__device__ __forceinline__ bool wait_xcds(const Buf& sb, int word, uint32_t want, int lane) {
   for (uint32_t spins = 1;; spins++) {
     const uint32_t v = sb.ld1(4u * (uint32_t)(word + (lane & (NXCD - 1))));
     if (__ballot((int)(v - want) < 0) == 0) return true;
     asm volatile("" ::: "memory");  // (every round loads)
-    if ((spins & 1023u) == 0 && give_up(sb, err, spins)) return false;
+    if ((spins & 1023u) == 0 && give_up(sb, spins)) return false;
   }
 }
 template <bool ANY>
@@ -330,12 +328,12 @@ __device__ __forceinline__ uint32_t settle_mode(const Buf& sb, uint32_t* sync, u
   }
 }
 // The other workgroups' wait for it (0: given up)
-__device__ __forceinline__ uint32_t wait_mode(const Buf& sb, uint32_t* err) {
+__device__ __forceinline__ uint32_t wait_mode(const Buf& sb) {
   for (uint32_t spins = 1;; spins++) {
     const uint32_t m = __builtin_amdgcn_readfirstlane(sb.ld1(4u * SY_MODE));
     if (m != 0u) return m;
     asm volatile("" ::: "memory");  // (every round loads)
-    if ((spins & 1023u) == 0 && give_up(sb, err, spins)) return 0u;
+    if ((spins & 1023u) == 0 && give_up(sb, spins)) return 0u;
   }
 }
 
@@ -344,8 +342,8 @@ __device__ __forceinline__ uint32_t wait_mode(const Buf& sb, uint32_t* err) {
 // step, wave and XCD), and when all XCDs' are done it tells its own workgroups. So a word that
 // crosses XCDs has one writer and eight readers; with every task storing a device-scope flag of
 // its own and every waiting workgroup polling them, a hand-over took 1.5-4 us (16 tokens).
-__device__ __forceinline__ void relay(const Buf& sb, const Buf& lb, uint32_t* err, const Sync& F, int nb, int G,
-                                      int layers, int wv, int lane) {
+__device__ __forceinline__ void relay(const Buf& sb, const Buf& lb, const Sync& F, int nb, int G, int layers, int wv,
+                                      int lane) {
   const int rb = wv * G, blocks = min(G, nb - rb);
   if (blocks <= 0) return;
   for (int l = 1; l <= layers; l++)
@@ -356,10 +354,10 @@ __device__ __forceinline__ void relay(const Buf& sb, const Buf& lb, uint32_t* er
       else if (s == S_O) word = F.o + rb * NO, n = NO * blocks;
       else if (s == S_GU) word = F.gu + rb * NGU, n = NGU * blocks;
       else word = F.down + rb * ND, n = ND * blocks;
-      if (!wait_local<false>(lb, sb, err, word + lane, lane < n, (uint32_t)l)) return;
+      if (!wait_local<false>(lb, sb, word + lane, lane < n, (uint32_t)l)) return;
       const int line = F.steps + (s * NW + wv) * SY_LINE;
       if (lane == 0) sb.st1((uint32_t)l, 4u * (uint32_t)line);
-      if (!wait_xcds(sb, err, line & ~(SY_LINE - 1), (uint32_t)l, lane)) return;
+      if (!wait_xcds(sb, line & ~(SY_LINE - 1), (uint32_t)l, lane)) return;
       if (lane == 0) store_local<false>(lb, F.relay + s * NW + wv, (uint32_t)l);
     }
 }
@@ -367,7 +365,8 @@ __device__ __forceinline__ void relay(const Buf& sb, const Buf& lb, uint32_t* er
 // Embedding rows of the prompt (an id outside the vocabulary sets the error word and reads row
 // 0) and the sync area cleared for the launch that follows.
 __global__ void __launch_bounds__(128) embed_rows_sync(const int* ids, const uint16_t* emb, uint16_t* h, uint32_t* err,
-                                                       uint32_t* sync, int nsync, uint32_t* local, int nlocal) {
+                                                       uint32_t* sync, int nsync, uint32_t* local, int nlocal,
+                                                       uint32_t dead) {
   const int s = blockIdx.x;
   int id = ids[s];
   if (id < 0 || id >= VOCAB) {
@@ -376,7 +375,7 @@ __global__ void __launch_bounds__(128) embed_rows_sync(const int* ids, const uin
   }
   reinterpret_cast<u32x4*>(h + (size_t)s * H)[threadIdx.x] = ldw(emb + (size_t)id * H + 8 * threadIdx.x);
   if (s == 0) {
-    for (int i = threadIdx.x; i < nsync; i += 128) sync[i] = 0u;
+    for (int i = threadIdx.x; i < nsync; i += 128) sync[i] = i == SY_DEAD ? dead : 0u;
     for (int i = threadIdx.x; i < nlocal; i += 128) local[i] = 0u;
   }
 }
@@ -451,8 +450,8 @@ __device__ __forceinline__ bool run_tasks(const ShortArgs& P, Shared& sm, int g,
     // every wave is done loading weights, and the tasks this one reads from are done
     auto ready = [&](int word, bool mine, uint32_t want) {
       if (wv == 0) {
-        if (!placed) placed = wait_mode(sb, P.err) == MODE_XCD;
-        const bool r = placed && wait_local<ANY>(lb, sb, P.err, word, mine, want);
+        if (!placed) placed = wait_mode(sb) == MODE_XCD;
+        const bool r = placed && wait_local<ANY>(lb, sb, word, mine, want);
         if (lane == 0) sm.ok = r;
       }
       __syncthreads();
@@ -781,7 +780,7 @@ __global__ void __launch_bounds__(NT) prefill_short(ShortArgs P) {
   if (!first && run_tasks<false>(P, sm, g, wv)) return;
   __syncthreads();
   if (wv == 0) {
-    const uint32_t m = first ? settle_mode(sb, P.sync, P.place_ticks, threadIdx.x & 63) : wait_mode(sb, P.err);
+    const uint32_t m = first ? settle_mode(sb, P.sync, P.place_ticks, threadIdx.x & 63) : wait_mode(sb);
     if (threadIdx.x == 0) sm.ok = m;
   }
   __syncthreads();
@@ -789,20 +788,20 @@ __global__ void __launch_bounds__(NT) prefill_short(ShortArgs P) {
     run_tasks<true>(P, sm, 0, wv);
   } else if (first) {
     const int nb = (P.S + 15) / 16;
-    relay(sb, Buf(P.local), P.err, Sync(nb, g), nb, (nb + NW - 1) / NW, P.num_layers, wv, threadIdx.x & 63);
+    relay(sb, Buf(P.local), Sync(nb, g), nb, (nb + NW - 1) / NW, P.num_layers, wv, threadIdx.x & 63);
   }
 }
 
 }  // namespace ps
 
-int prefill_short_run(const int* ids, const uint16_t* embed, const ps::ShortArgs& A, bool any_xcd, hipStream_t stream) {
+int prefill_short_run(const int* ids, const uint16_t* embed, const ps::ShortArgs& A, int debug, hipStream_t stream) {
   const int nb = (A.S + 15) / 16;
   ps::embed_rows_sync<<<A.S, 128, 0, stream>>>(ids, embed, A.h, A.err, A.sync, ps::SYNC_WORDS, A.local,
-                                               ps::NXCD * ps::local_words(nb));
+                                               ps::NXCD * ps::local_words(nb), debug & MQ_DEBUG_PREFILL_GAVE_UP ? 1u : 0u);
   if (hipGetLastError() != hipSuccess) return MQ_ERR_HIP;
   ps::ShortArgs B = A;
   B.groups = nb < ps::GROUPS ? nb : ps::GROUPS;
-  B.place_ticks = any_xcd ? 0 : ps::PLACE_TICKS;
+  B.place_ticks = debug & MQ_DEBUG_PREFILL_ANY_XCD ? 0 : ps::PLACE_TICKS;
   ps::prefill_short<<<ps::NWG, ps::NT, 0, stream>>>(B);
   return hipGetLastError() == hipSuccess ? MQ_OK : MQ_ERR_HIP;
 }

@@ -137,8 +137,8 @@ class MegakernelDecoder:
             # goes back to before the step, so the next step rewrites them.
             self.position_ = position_before
             _abi.lib().mq_reset_workspace(self._device())
-            raise _abi.MegakernelError(f"kernel reported error flags {-tok - 1} (decode watchdog, or a prompt id "
-                                       f"out of range in prefill); workspace reset, position restored to "
+            raise _abi.MegakernelError(f"kernel reported error flags {-tok - 1} (decode watchdog; or in prefill "
+                                       f"1: a prompt id out of range, 2: a wait given up); workspace reset, position restored to "
                                        f"{position_before}")
         return tok
 

@@ -102,13 +102,13 @@ def _prefill_args(**over):
 def test_prefill_rejects_invalid_arguments(bad):
     keep, args = _prefill_args(**bad)
     assert _abi.lib().launch_prefill_float(*args) == _abi.MQ_ERR_ARG
-    assert _abi.lib().mq_debug_prefill_any_xcd(*args) == _abi.MQ_ERR_ARG
+    assert _abi.lib().mq_debug_prefill(0, *args) == _abi.MQ_ERR_ARG
     del keep
 
 
 def test_single_list_prefill_hook_rejects_long_prompts():
     keep, args = _prefill_args(seq_len=257, max_seq_len=512)
-    assert _abi.lib().mq_debug_prefill_any_xcd(*args) == _abi.MQ_ERR_ARG
+    assert _abi.lib().mq_debug_prefill(0, *args) == _abi.MQ_ERR_ARG
     del keep
 
 

@@ -7,6 +7,8 @@ residual stream after the last layer. The ragged-length tests of test_gpu_prefil
 both paths with the numpy oracle.
 """
 
+from functools import partial
+
 import pytest
 import torch
 
@@ -17,6 +19,7 @@ from megaqwen_amd import rope, weights
 pytestmark = pytest.mark.gpu
 
 N_LAYERS, LONG = 3, 300
+ANY_XCD, GAVE_UP = 1, 2  # MQ_DEBUG_PREFILL_*
 
 
 @pytest.fixture(scope="module")
@@ -77,7 +80,7 @@ def test_single_list_gives_the_same_bits(models, S, monkeypatch):
     """The form for launches whose workgroups cannot be on every XCD at once (forced from the
     host): tasks from one list, every hand-over device-wide."""
     (dec, _), ids, want = models
-    monkeypatch.setattr(_abi.lib(), "launch_prefill_float", _abi.lib().mq_debug_prefill_any_xcd)
+    monkeypatch.setattr(_abi.lib(), "launch_prefill_float", partial(_abi.lib().mq_debug_prefill, ANY_XCD))
     print(f"prefill S={S}", flush=True)
     for rep in range(2):
         dec.reset()
@@ -86,3 +89,24 @@ def test_single_list_gives_the_same_bits(models, S, monkeypatch):
             ref = ref[:, :, :S] if name in "kv" else ref[:S]
             assert torch.equal(got, ref), (name, rep)
         assert not dec.k_cache_[:, :, S:].any() and not dec.v_cache_[:, :, S:].any()
+
+
+@pytest.mark.parametrize("failing", [0, 1])
+def test_a_launch_that_gives_up_says_so_itself(models, failing, monkeypatch):
+    """The give-up word belongs to the launch that set it (forced from the host): its own result is
+    -3, a prefill beside it returns its token, whichever comes first."""
+    decs, ids, _ = models
+    lib, S = _abi.lib(), 40
+    token = decs[0].prefill_step(ids[:S])
+    normal, gave_up = lib.launch_prefill_float, partial(lib.mq_debug_prefill, GAVE_UP)
+    print("prefill S=40, give-up word set", flush=True)
+    for i, dec in enumerate(decs):
+        monkeypatch.setattr(lib, "launch_prefill_float", gave_up if i == failing else normal)
+        dec.prefill_step_async(ids[:S])
+    got = [int(dec.output_token_.item()) for dec in decs]
+    assert got[failing] == -3 and got[1 - failing] == token
+    monkeypatch.setattr(lib, "launch_prefill_float", gave_up)
+    with pytest.raises(_abi.MegakernelError, match="error flags 2"):
+        decs[0].prefill_step(ids[:S])
+    monkeypatch.setattr(lib, "launch_prefill_float", normal)
+    assert decs[0].position() == 0 and decs[0].prefill_step(ids[:S]) == token
