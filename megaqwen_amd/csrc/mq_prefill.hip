@@ -108,8 +108,8 @@ struct QknArgs {
 struct XcdMap {
   int xg, xp;
 };
-// Cache warm-up by workgroups that no tile uses. A launch that leaves CUs idle (gate/up at
-// S = 512 has 192 workgroups for 256 CUs) appends one row of workgroups (blockIdx.y ==
+// Cache warm-up by workgroups that no tile uses. A launch that leaves CUs idle (gate/up up to
+// 384 tokens has at most 192 workgroups for 256 CUs) appends one row of workgroups (blockIdx.y ==
 // `row`) that read the weights of the launches after it, each column tile of a consumer on
 // the XCD that will read it: in blockIdx order with a multiple of 8 column tiles, a
 // consumer's column tile t runs on XCD t % 8 whatever its row tile and k split. Nothing is
@@ -120,9 +120,8 @@ struct XcdMap {
 // prefill, same box: S = 300 1.779 -> 1.807 ms, 512 1.962 -> 1.992).
 constexpr int MAX_WARM = 5, NUM_CUS = 256;  // (MI355X: 8 XCDs of 32 CUs)
 // Prompts up to this length warm in gate/up (whole prefill, same box, without -> with the
-// warm-up: S = 288 1.755 -> 1.730 ms, 352 1.804 -> 1.760, 384 1.839 -> 1.782; from 385 tokens
-// gate/up has 192 tile workgroups, and with the warm-up row S = 400 measured 1.794 -> 1.801, 512
-// 1.930 -> 1.927)
+// warm-up: S = 257 1.699 -> 1.669 ms, 300 1.748 -> 1.711, 352 1.791 -> 1.741, 384 1.823 -> 1.758; from
+// 385 tokens gate/up's own 256 tiles fill the CUs)
 constexpr int WARM_MAX_S = 384;
 struct WarmSet {
   const uint16_t* w[MAX_WARM];  // weight matrices [n, k] bf16, in the order they are read
@@ -1309,6 +1308,7 @@ __global__ void __launch_bounds__(64 * F2W) attn_prefill_fa2(const uint16_t* q, 
 // number of DMAs before each wait and the vmcnt count stays exact.
 // waves, heads a wave, query rows, ring, DMAs per item and wave
 constexpr int F3W = 4, F3H = 1, F3Q = 16 * F3W * F3H / 2, F3R = 4, F3I = 4;
+static_assert(F3H == 1, "a wave's rows and head (wr and h0 in attn_prefill_fa3) are those of one head a wave");
 // A block's scores are parked in accumulation registers (AGPRs) once the maxima have read
 // them, and brought back to VGPRs chunk by chunk for the exponentials (an empty asm with an
 // AGPR / VGPR operand: the compiler moves the value there), so that the 128 registers of
@@ -1794,7 +1794,7 @@ static void gemm_qkv(GemmArgs g, hipStream_t stream) {
 }
 // warm: the warm-up set of a prompt of at most WARM_MAX_S tokens, or null
 static void gemm_gate_up(GemmArgs g, hipStream_t stream, const WarmSet* warm = nullptr) {
-  static_assert(WARM_MAX_S <= 512, "the warm-up set's column tiles are those of the shapes up to 512 tokens");
+  static_assert(WARM_MAX_S <= 512, "the warm-up set's column tiles are those of the shapes up to 512 tokens, and only they take it");
   if (g.m > 640) {
     // 24 column tiles of 128 units, and the row tile that fills the rounds of 256 workgroups best.
     // The launch alone with one tile for each range before (128 and 256 rows) -> now, same box,
@@ -1815,7 +1815,7 @@ static void gemm_gate_up(GemmArgs g, hipStream_t stream, const WarmSet* warm = n
     }
   } else if (g.m > 512) {
     g.seg[0].ntiles = I / 64;
-    gemm<EPI_SILU, 128, 128, 3, 1, 4, 4>(g, I / 64, stream, 1, 0, 1, warm);
+    gemm<EPI_SILU, 128, 128, 3, 1, 4, 4>(g, I / 64, stream);
   } else {
     // (257..512 tokens: 128 x 96 tiles on four waves, 64 column tiles, so 256 workgroups fill
     // the CUs where the 128 x 128 tiles leave 64 idle; same bits, whole prefill, same box:
@@ -1829,12 +1829,13 @@ static void gemm_gate_up(GemmArgs g, hipStream_t stream, const WarmSet* warm = n
 // o_proj / down_proj with the residual add in the epilogue (the four k quarters summed in order
 // inside the workgroup: the same bits as the split-four partials and resid_norm_rows); out = h,
 // updated in place. The fp32 partials cost 32 bytes an output written and read again where h costs 4,
-// but they let four times the workgroups run: this form starts where 128-row tiles fill the CUs
-// better than half (tiles of 32 to 64 rows for shorter prompts are even with the partials alone and
-// lose 1-3% in the whole prefill, whose weights and activations are cold). Launch and the norm after
+// but a workgroup then walks only a quarter of k (around the line 144 workgroups of 256 x 256 tiles
+// against 136 or 144 of 128 x 128 with all of k). The line is where the whole prefill says: partials ->
+// this form, same box, ms, S = 2049 5.243 -> 5.288, 2112 5.343 -> 5.371, 2176 5.451 -> 5.494, 2177 5.457 -> 5.431, 2240 5.550 -> 5.520 (a
+// second box -0.5% and +1.8% on the two sides of it). Tiles of 32 to 64 rows for shorter prompts are
+// even with the partials alone and lose 1-3% in the whole prefill, whose weights and activations are cold. Launch and the norm after
 // it, partials -> this form, us: S = 3000 33.5 -> 24.9 and 40.3 -> 31.9, 6000 62.1 -> 37.8 and 75.9 ->
-// 50.9. Whole prefill, same box, partials -> this form, ms: S = 2049 5.797 -> 5.836, 2200 6.019 -> 6.000, 3000
-// 7.44 -> 7.27, 4300 11.96 -> 11.38, 5400 15.50 -> 14.54, 6000 16.70 -> 15.64, 7000 19.41 -> 18.57.
+// 50.9. Whole prefill, same box, partials -> this form, ms: S = 3000 7.44 -> 7.27, 4300 11.96 -> 11.38, 5400 15.50 -> 14.54, 6000 16.70 -> 15.64, 7000 19.41 -> 18.57.
 constexpr int RESADD_MIN_S = 2177;
 static void gemm_residual_add(GemmArgs g, uint16_t* h, hipStream_t stream) {
   // 8 column tiles, the row tile by rounds of workgroups (o_proj and down_proj together, us a round;
@@ -1856,7 +1857,8 @@ static void gemm_residual_add(GemmArgs g, uint16_t* h, hipStream_t stream) {
 // o_proj / down_proj as four k splits of fp32 partials, below RESADD_MIN_S tokens
 static void gemm_residual(GemmArgs g, hipStream_t stream) {
   if (g.m > 2048) {
-    // (one round where the 128 x 256 tiles need two)
+    // (up to 2176 tokens one round where the 128 x 256 tiles need two: whole prefill, same box, ms, S =
+    // 2049 5.393 -> 5.130, 2112 5.520 -> 5.212, 2176 5.605 -> 5.326)
     g.seg[0].ntiles = H / 256;
     gemm<EPI_PART, 256, 256, 2, 1, 4, 4>(g, H / 256, stream, RES_SPLIT);
   } else if (g.m > 1536) {
