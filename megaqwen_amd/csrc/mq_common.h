@@ -81,6 +81,11 @@ __device__ __forceinline__ f32x4 mfma_16x16x32(const u32x4& a, const u32x4& b, f
                                                   0, 0);
 }
 
+// exp(x) as 2^(x log2 e) on the hardware exp2 (v_exp_f32): about 2^-20 relative error for
+// the arguments of the softmax (x <= 0), the accuracy class of the vectorised exp that
+// torch's CPU flash-attention kernel uses (exp_u20); exp(-inf) = 0.
+__device__ __forceinline__ float exp_fast(float x) { return __builtin_amdgcn_exp2f(x * 1.44269504088896341f); }
+
 // ------------------------------------------------------------------ wave64 reductions
 // DPP row operations (16-lane rows): quad_perm [1,0,3,2] and [2,3,0,1] pair
 // lanes within quads, row_half_mirror pairs lane i with 7-i, row_mirror lane i
@@ -209,6 +214,18 @@ __device__ __forceinline__ u32x4 ldw(const uint16_t* p) { return __builtin_nonte
 __device__ __forceinline__ u32x2 ldw2(const uint16_t* p) { return __builtin_nontemporal_load((gu32x2*)(p)); }
 __device__ __forceinline__ uint32_t ldw1(const uint16_t* p) { return __builtin_nontemporal_load((gu32*)(p)); }
 __device__ __forceinline__ uint32_t ldraw16(const uint16_t* p) { return *(gu16*)(p); }
+
+// Embedding row of prompt token s, copied by 128 threads. An id outside the vocabulary sets the
+// error word (reported as a negative token) and reads row 0.
+__device__ __forceinline__ void embed_row(const int* ids, const uint16_t* emb, uint16_t* h, uint32_t* err, int s,
+                                          int thread) {
+  int id = ids[s];
+  if (id < 0 || id >= VOCAB) {
+    if (thread == 0) __hip_atomic_fetch_or(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    id = 0;
+  }
+  reinterpret_cast<u32x4*>(h + (size_t)s * H)[thread] = ldw(emb + (size_t)id * H + 8 * thread);
+}
 
 // A pointer that is the same in every lane, moved to scalar registers.
 template <typename T>

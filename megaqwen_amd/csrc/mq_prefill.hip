@@ -587,16 +587,9 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_nt_warm(KernArgs<EPI> G, Wa
 }
 
 // ------------------------------------------------------------------ row-wise kernels
-// Embedding rows of the prompt. An id outside the vocabulary sets the error word
-// (reported as a negative token) and reads row 0.
+// Embedding rows of the prompt.
 __global__ void __launch_bounds__(128) embed_rows(const int* ids, const uint16_t* emb, uint16_t* h, uint32_t* err) {
-  const int s = blockIdx.x;
-  int id = ids[s];
-  if (id < 0 || id >= VOCAB) {
-    if (threadIdx.x == 0) __hip_atomic_fetch_or(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    id = 0;
-  }
-  reinterpret_cast<u32x4*>(h + (size_t)s * H)[threadIdx.x] = ldw(emb + (size_t)id * H + 8 * threadIdx.x);
+  embed_row(ids, emb, h, err, blockIdx.x, threadIdx.x);
 }
 
 // HF Qwen3RMSNorm (modeling_qwen3.py:59-64) of each row: y = bf16(w * bf16(x * rstd)),
@@ -733,10 +726,6 @@ constexpr int SC_PITCH = AKB + 1, P_PITCH = AKB + 8;
 
 __device__ __forceinline__ uint32_t akv_off(int row, int chunk) { return row * 256 + 16 * (chunk ^ (row & 15)); }
 
-// exp(x) as 2^(x log2 e) on the hardware exp2 (v_exp_f32): about 2^-20 relative error for
-// the arguments of the softmax (x <= 0), the accuracy class of the vectorised exp that
-// torch's CPU flash-attention kernel uses (exp_u20); exp(-inf) = 0.
-__device__ __forceinline__ float exp_fast(float x) { return __builtin_amdgcn_exp2f(x * 1.44269504088896341f); }
 // x, opaque to the compiler: a product passed through it is rounded on its own and never
 // contracted with a later add into one fused multiply-add
 __device__ __forceinline__ float unfused(float x) {
@@ -1831,11 +1820,12 @@ static void gemm_gate_up(GemmArgs g, hipStream_t stream, const WarmSet* warm = n
 // updated in place. The fp32 partials cost 32 bytes an output written and read again where h costs 4,
 // but a workgroup then walks only a quarter of k (around the line 144 workgroups of 256 x 256 tiles
 // against 136 or 144 of 128 x 128 with all of k). The line is where the whole prefill says: partials ->
-// this form, same box, ms, S = 2049 5.243 -> 5.288, 2112 5.343 -> 5.371, 2176 5.451 -> 5.494, 2177 5.457 -> 5.431, 2240 5.550 -> 5.520 (a
-// second box -0.5% and +1.8% on the two sides of it). Tiles of 32 to 64 rows for shorter prompts are
-// even with the partials alone and lose 1-3% in the whole prefill, whose weights and activations are cold. Launch and the norm after
-// it, partials -> this form, us: S = 3000 33.5 -> 24.9 and 40.3 -> 31.9, 6000 62.1 -> 37.8 and 75.9 ->
-// 50.9. Whole prefill, same box, partials -> this form, ms: S = 3000 7.44 -> 7.27, 4300 11.96 -> 11.38, 5400 15.50 -> 14.54, 6000 16.70 -> 15.64, 7000 19.41 -> 18.57.
+// this form, same box, ms, S = 2049 5.243 -> 5.288, 2112 5.343 -> 5.371, 2176 5.451 -> 5.494, 2177
+// 5.457 -> 5.431, 2240 5.550 -> 5.520 (a second box -0.5% and +1.8% on the two sides of it), 3000 7.44 ->
+// 7.27, 4300 11.96 -> 11.38, 5400 15.50 -> 14.54, 6000 16.70 -> 15.64, 7000 19.41 -> 18.57. Launch and the
+// norm after it, us: S = 3000 33.5 -> 24.9 and 40.3 -> 31.9, 6000 62.1 -> 37.8 and 75.9 -> 50.9. Tiles of 32
+// to 64 rows for shorter prompts are even with the partials alone and lose 1-3% in the whole prefill,
+// whose weights and activations are cold.
 constexpr int RESADD_MIN_S = 2177;
 static void gemm_residual_add(GemmArgs g, uint16_t* h, hipStream_t stream) {
   // 8 column tiles, the row tile by rounds of workgroups (o_proj and down_proj together, us a round;

@@ -362,26 +362,16 @@ __device__ __forceinline__ void relay(const Buf& sb, const Buf& lb, const Sync& 
     }
 }
 
-// Embedding rows of the prompt (an id outside the vocabulary sets the error word and reads row
-// 0) and the sync area cleared for the launch that follows.
+// Embedding rows of the prompt, and the sync area cleared for the launch that follows.
 __global__ void __launch_bounds__(128) embed_rows_sync(const int* ids, const uint16_t* emb, uint16_t* h, uint32_t* err,
                                                        uint32_t* sync, int nsync, uint32_t* local, int nlocal,
                                                        uint32_t dead) {
-  const int s = blockIdx.x;
-  int id = ids[s];
-  if (id < 0 || id >= VOCAB) {
-    if (threadIdx.x == 0) __hip_atomic_fetch_or(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    id = 0;
-  }
-  reinterpret_cast<u32x4*>(h + (size_t)s * H)[threadIdx.x] = ldw(emb + (size_t)id * H + 8 * threadIdx.x);
-  if (s == 0) {
+  embed_row(ids, emb, h, err, blockIdx.x, threadIdx.x);
+  if (blockIdx.x == 0) {
     for (int i = threadIdx.x; i < nsync; i += 128) sync[i] = i == SY_DEAD ? dead : 0u;
     for (int i = threadIdx.x; i < nlocal; i += 128) local[i] = 0u;
   }
 }
-
-// exp(x) as 2^(x log2 e) (mq_prefill.hip's exp_fast)
-__device__ __forceinline__ float exp_fast(float x) { return __builtin_amdgcn_exp2f(x * 1.44269504088896341f); }
 
 constexpr int MAXK = SHORT_MAX_S;             // keys of the longest prompt
 constexpr int SC_PITCH = MAXK + 4;            // score row pitch (floats); the row's probabilities overlay it
