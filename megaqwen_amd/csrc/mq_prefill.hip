@@ -1279,7 +1279,7 @@ __global__ void __launch_bounds__(64 * F2W) attn_prefill_fa2(const uint16_t* q, 
 // are short enough to fill the CUs. Both heads' rows in one wave (64-row blocks, 432 registers,
 // one wave a SIMD) read K and V from LDS half as often and were slower at every length, with the
 // same bits: S = 1024 33.8 -> 26.7 us, 1117 36.8 -> 29.5, 1536 48.5 -> 39.5, 3000 90.2 -> 75.1, 5000
-// 215 -> 179. The operations and their order are those of
+// 215 -> 179 (both timed with the one-rounding exponent below; with this one 1117 30.7, 3000 82.5). The operations and their order are those of
 // attn_prefill_fa2 (scores, maxima, exponentials, in-lane sums, P.V chains, rescaling), so the
 // two give the same bits; this one does a third less MFMA work and reads K from LDS once per block
 // instead of twice. (The exponent with one rounding, exp2(fma(a, scale log2 e, -max log2 e)),
