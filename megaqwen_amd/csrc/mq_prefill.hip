@@ -1821,7 +1821,7 @@ static void gemm_gate_up(GemmArgs g, hipStream_t stream, const WarmSet* warm = n
 // but a workgroup then walks only a quarter of k (around the line 144 workgroups of 256 x 256 tiles
 // against 136 or 144 of 128 x 128 with all of k). The line is where the whole prefill says: partials ->
 // this form, same box, ms, S = 2049 5.243 -> 5.288, 2112 5.343 -> 5.371, 2176 5.451 -> 5.494, 2177
-// 5.457 -> 5.431, 2240 5.550 -> 5.520 (a second box -0.5% and +1.8% on the two sides of it), 3000 7.44 ->
+// 5.457 -> 5.431, 2240 5.550 -> 5.520 (another card -0.5% and +1.8% on the two sides of it), 3000 7.44 ->
 // 7.27, 4300 11.96 -> 11.38, 5400 15.50 -> 14.54, 6000 16.70 -> 15.64, 7000 19.41 -> 18.57. Launch and the
 // norm after it, us: S = 3000 33.5 -> 24.9 and 40.3 -> 31.9, 6000 62.1 -> 37.8 and 75.9 -> 50.9. Tiles of 32
 // to 64 rows for shorter prompts are even with the partials alone and lose 1-3% in the whole prefill,

@@ -56,8 +56,8 @@ def test_short_prompt_equals_the_long_prompts_rows(models, S):
 
 
 def test_short_prompts_on_two_streams(models):
-    """Launches of two decoders overlap on two streams: each has its own sync words and makes
-    progress with the workgroups that the other leaves it."""
+    """Launches of two decoders that may overlap on two streams: each has its own sync words, and one
+    that does not find workgroups of its own on every XCD runs from a single list."""
     decs, ids, want = models
     streams = [torch.cuda.Stream() for _ in decs]
     lengths = (128, 40)
